@@ -188,8 +188,9 @@ namespace {
 
 // Kernel variant of a request: KIND, interleaved fields NFP, record mode and
 // MODE (VR: bit 0 ColorTransferFunction path, bit 1 n_samples == 10, bit 2
-// early ray termination, bit 3 per-pixel lens; projection: bit 3).  NFP 4
-// and 8 variants keep only bits 0 and 3.
+// early ray termination, bit 3 per-pixel lens, bit 4 vertex blocks in LDS,
+// bit 5 with bit 0 grey opacity (one field, no bit 2); projection: bit 3).
+// NFP 4 and 8 variants keep only bits 0 and 3.
 // Sampler kinds that read a transfer function.
 inline bool has_tf(int kind) { return kind == YTRC_VOLUME_RENDER || kind == YTRC_LIGHT_SOURCE; }
 
@@ -244,7 +245,8 @@ pfn_t pick_persist(int kind, int nfp, bool rec, int mode)
     if (m < 2) return pick_persist_vr_a(nfp, rec, m);
     if (m < 4 || m == 19) return pick_persist_vr_b(nfp, rec, m);
     if (m < 8) return pick_persist_vr_c(nfp, rec, m);
-    return pick_persist_vr_d(nfp, rec, m);
+    if (m < 16) return pick_persist_vr_d(nfp, rec, m);
+    return pick_persist_vr_e(nfp, rec, m);
 }
 
 kfn_t pick_kernel(int kind, int nfp, bool rec, int mode)
@@ -257,7 +259,8 @@ kfn_t pick_kernel(int kind, int nfp, bool rec, int mode)
     if (m < 2) return pick_kernel_vr_a(nfp, rec, m);
     if (m < 4) return pick_kernel_vr_b(nfp, rec, m);
     if (m < 8) return pick_kernel_vr_c(nfp, rec, m);
-    return pick_kernel_vr_d(nfp, rec, m);
+    if (m < 16) return pick_kernel_vr_d(nfp, rec, m);
+    return pick_kernel_vr_e(nfp, rec, m);
 }
 
 }  // namespace
@@ -962,6 +965,47 @@ struct PrepReq {
     int tsh = TILE_SHIFT_DEFAULT;
 };
 
+// An upper bound of the t-interval of any ray of the request in one cell.
+double longest_cell_interval(const ytrc_request &r, const Dataset &ds, bool per_pixel)
+{
+    double tcell = 0.0;
+    if (!per_pixel) {
+        for (int k = 0; k < r.n_order; k++) {
+            const DBrick &hb = ds.h_bricks[r.order[k]];
+            double cmin = 1.0;
+            for (int a = 0; a < 3; a++)
+                if (r.vp_dir[a] != 0.0) cmin = std::min(cmin, hb.dds[a] / std::fabs(r.vp_dir[a]));
+            tcell = std::max(tcell, cmin);
+        }
+        return tcell;
+    }
+    // Any chord of a cell is at most its diagonal: the longest in-cell
+    // t-interval is below diag / |v_dir| over all rays.
+    double dmin = 1e300, diag = 0.0;
+    for (int64_t p = 0; p < (int64_t)r.nv[0] * r.nv[1]; p++) {
+        const double *v = r.pix_dir + 3 * p;
+        dmin = std::min(dmin, std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
+    }
+    for (int k = 0; k < r.n_order; k++) {
+        const DBrick &hb = ds.h_bricks[r.order[k]];
+        diag = std::max(diag, std::sqrt(hb.dds[0] * hb.dds[0] + hb.dds[1] * hb.dds[1] + hb.dds[2] * hb.dds[2]));
+    }
+    return dmin > 0.0 ? diag / dmin : HUGE_VAL;
+}
+
+// The grey compositing of ctf_visit_grey: every table value finite and dt *
+// alpha <= 1 for sub-samples of length dt at most dt_max.
+bool grey_bounded(const ytrc_tf_desc &tf, double dt_max)
+{
+    double amax = 0.0;
+    for (int t = 0; t < 4; t++)
+        for (int k = 0; k < tf.nbins[t]; k++) {
+            if (!std::isfinite((float)tf.y[t][k])) return false;
+            if (t == 3) amax = std::max(amax, std::fabs(tf.y[t][k]));
+        }
+    return std::isfinite(dt_max) && amax * dt_max * 1.001 <= 1.0;
+}
+
 int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, PrepReq &P,
                  int tsh = TILE_SHIFT_DEFAULT)
 {
@@ -1109,8 +1153,10 @@ int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, P
         // Transmittance-form compositing is exact when every sub-sample has
         // a = dt * e <= 1: bound e by the tables' largest magnitudes and dt
         // by the longest in-cell t-interval / n_samples.
+        double tcell = 0.0;
+        if (!T.grey || ctf) tcell = longest_cell_interval(r, ds, pp);
         if (!T.grey) {
-            bool bounded = true;
+            bool bounded = std::isfinite(tcell);
             double emax = 0.0;
             for (int t = 0; t < tf.n_fits; t++) bounded = bounded && tf.weight_field_ids[t] == -1;
             for (int c = 0; bounded && c < 3; c++) {
@@ -1124,37 +1170,19 @@ int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, P
                 }
                 emax = std::max(emax, ec);
             }
-            double tcell = 0.0;
-            if (!pp) {
-                for (int k2 = 0; bounded && k2 < r.n_order; k2++) {
-                    const DBrick &hb = ds.h_bricks[r.order[k2]];
-                    double cmin = 1.0;
-                    for (int a = 0; a < 3; a++)
-                        if (r.vp_dir[a] != 0.0) cmin = std::min(cmin, hb.dds[a] / std::fabs(r.vp_dir[a]));
-                    tcell = std::max(tcell, cmin);
-                }
-            } else {
-                // Any chord of a cell is at most its diagonal: the longest
-                // in-cell t-interval is below diag / |v_dir| over all rays.
-                double dmin = 1e300, diag = 0.0;
-                for (int64_t p = 0; p < (int64_t)r.nv[0] * r.nv[1]; p++) {
-                    const double *v = r.pix_dir + 3 * p;
-                    dmin = std::min(dmin, std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
-                }
-                for (int k2 = 0; k2 < r.n_order; k2++) {
-                    const DBrick &hb = ds.h_bricks[r.order[k2]];
-                    diag = std::max(diag, std::sqrt(hb.dds[0] * hb.dds[0] + hb.dds[1] * hb.dds[1] +
-                                                    hb.dds[2] * hb.dds[2]));
-                }
-                tcell = dmin > 0.0 ? diag / dmin : 1e300;
-                bounded = bounded && std::isfinite(tcell);
-            }
             q.tform = bounded && (emax * (tcell / (double)r.n_samples) * 1.001 <= 1.0);
         }
         // ColorTransferFunction pattern (transfer_functions.py:385-408) in
         // transmittance form gets its own kernel path (MODE bit 0); grey or
         // unbounded CTFs take the general per-table path.
-        ctf = ctf && q.tform && r.kind == YTRC_VOLUME_RENDER;
+        // Grey opacity on one field without early termination or partial maps
+        // gets its own layout and compositing (MODE bits 0 and 5,
+        // ctf_visit_grey) where dt * alpha <= 1 holds for every sub-sample by
+        // the same bound, so that the reference's clamp of 1 - dt alpha never
+        // acts, and the tables are finite.
+        const bool grey = ctf && T.grey && r.kind == YTRC_VOLUME_RENDER && q.nfp == 1 &&
+                          !(r.flags & (YTRC_FLAG_ERT | YTRC_FLAG_PARTIAL)) && grey_bounded(tf, tcell / (double)r.n_samples);
+        ctf = (ctf && q.tform && r.kind == YTRC_VOLUME_RENDER) || grey;
         if (ctf) {
             // Transmittance form: per bin, the two lerps whose product is
             // the emission, e_c = (y_c + f dy_c)(y_a + f dy_a), c = r, g, b
@@ -1171,6 +1199,22 @@ int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, P
             // entries start on all 16 bank groups of the LDS rather than
             // every other one, which halves the bank conflicts of the
             // scattered per-lane reads.
+            // Grey opacity keeps the general tables' values: entry k + 1 of
+            // 48 bytes holds {y}, {dy} and d0 of bin k, entry 0 is zero
+            // (ctf_visit_grey).
+            const int nb = tf.nbins[0];
+            if (grey) {
+                std::vector<float4> lay((size_t)3 * nb, make_float4(0.f, 0.f, 0.f, 0.f));
+                for (int k = 0; k < nb - 1; k++) {
+                    const float4 *g = &P.tft[(size_t)k];
+                    lay[3 * k + 3] = make_float4(g[0].x, g[nb].x, g[2 * nb].x, g[3 * nb].x);
+                    lay[3 * k + 4] = make_float4(g[0].y, g[nb].y, g[2 * nb].y, g[3 * nb].y);
+                    lay[3 * k + 5].x = g[0].z;
+                }
+                P.tft = std::move(lay);
+            }
+        }
+        if (ctf && !grey) {
             const int nb = tf.nbins[0];
             const double b0 = tf.bounds[0], b1 = tf.bounds[1];
             const double idbin = 1.0 / ((b1 - b0) / (double)(nb - 1));
@@ -1194,7 +1238,7 @@ int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, P
             tot = (int)P.tft.size();
             T.mode = 1;
         }
-        q.mode = T.mode | (r.n_samples == 10 ? 2 : 0) |
+        q.mode = T.mode | (grey ? 32 : 0) | (r.n_samples == 10 ? 2 : 0) |
                  ((r.flags & (YTRC_FLAG_ERT | YTRC_FLAG_PARTIAL)) ? 4 : 0) | (pp ? 8 : 0);
         T.total_bins = tot;
         q.lds = (size_t)tot * sizeof(float4);

@@ -639,7 +639,51 @@ __device__ __forceinline__ void ctf_visit(const TFCache &tf, const float4 *__res
     for (int ch = 0; ch < 3; ch++) st[ch] = __builtin_fma(-st[ch], (double)Q[ch], st[ch]);
 }
 
+// The sub-samples of one visit for a ColorTransferFunction with grey opacity
+// (every channel attenuated by alpha): fit_eval_general's arithmetic on the
+// four tables, which share their bins, and the same FP64 compositing
+// (field_interpolation_tables.pxd:66-106), so the same values bit for bit.
+// One entry of 48 bytes per bin, {y}, {dy}, {d0} of the tables, is read with
+// two 16-byte and one 4-byte LDS reads instead of four 16-byte ones; entry 0
+// is zero and stands for every value outside (b0, b1) or not normal, entry k
+// + 1 for bin k.  The host has shown dt alpha <= 1 for every sub-sample, so
+// the reference's clamp of 1 - dt alpha at 0 never acts.  k: the value along
+// the visit's sub-samples, k0 + k1 s + k2 s^2 + k3 s^3.  About 20 FP32 and
+// 12 FP64 VALU per sub-sample bound it; with the general tables' 16 lookups'
+// worth of selects, 192^3 at 512^2 took 5.34 ms, now 1.00 ms.
+template <int NS>
+__device__ __forceinline__ void ctf_visit_grey(const TFCache &tf, const float4 *__restrict__ lt,
+                                               const float (&k)[4], double dt, int ns, double (&st)[4])
+{
+    const int nsq = (NS > 0) ? NS : ns;
+    float sf = 0.0f;
+    // (unrolled whole, the compiler gathers every sub-sample's reads first:
+    // 247 VGPRs; by 1 or 5 instead of 2: 5 to 10 % and 2 % slower)
+#pragma unroll 2
+    for (int s = 0; s < nsq; s++, sf += 1.0f) {
+        const float v = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(k[3], sf, k[2]), sf, k[1]), sf, k[0]);
+        const bool ok = (v < tf.b1) & (v > tf.b0) & __builtin_amdgcn_classf(v, (1 << 3) | (1 << 8));
+        const int bin = (int)((v - tf.b0) * tf.idbin);
+        const int at = ok ? min(bin, tf.nbm2) + 1 : 0;
+        const float4 *q = (const float4 *)((const char *)lt + __umul24((unsigned)at, 48u));
+        const float4 y = q[0], d = q[1];
+        // (an infinite v times the zero entry's 0 would be NaN)
+        const float x = ok ? v - *(const float *)(q + 2) : 0.0f;
+        const float a = __builtin_fmaf(x, d.w, y.w);
+        const float e0 = __builtin_fmaf(x, d.x, y.x) * a;
+        const float e1 = __builtin_fmaf(x, d.y, y.y) * a;
+        const float e2 = __builtin_fmaf(x, d.z, y.z) * a;
+        const double da = dt * (double)a;
+        const double ta = 1.0 - da;
+        st[0] = __builtin_fma(ta, st[0], dt * (double)e0);
+        st[1] = __builtin_fma(ta, st[1], dt * (double)e1);
+        st[2] = __builtin_fma(ta, st[2], dt * (double)e2);
+        st[3] = __builtin_fma(ta, st[3], da);
+    }
+}
+
 // VolumeRenderSampler.sample (image_samplers.pyx:453-487).
+// MODE bit 5 (with bit 0): the ColorTransferFunction has grey opacity.
 // MODE bit 0: ColorTransferFunction in transmittance form; bit 1: n_samples == 10 unrolled;
 // bit 2: early ray termination.
 // st[] is the compositing state: rgba, or, when `tform` is set (non-grey
@@ -679,12 +723,6 @@ struct VRSampler {
         } else {
             for (int s = 0; s < ns; s++) body(s);
         }
-    }
-
-    template <int NS>
-    __device__ __forceinline__ void ctf_samples(const float (&ku)[4], double dt, int ns)
-    {
-        ctf_visit<NS>(*tf, lt, ku, (float)dt, ns, st);
     }
 
     template <int NS>
@@ -749,6 +787,17 @@ struct VRSampler {
         const int mval = (mask != nullptr) ? (int)mask[cell] : 1;
         float cv[8][NFP];
         load_corners<NFP>(data + (size_t)voff * NFP, cv);
+        sample<(MODE & 32) == 0>(en, ex, (double)c0, (double)c1, (double)c2, cv, mval);
+    }
+
+    // The visit of cell (c0, c1, c2) (as doubles) whose mask byte and corner
+    // loads have been issued.  UNROLL: unroll n_samples == 10 (MODE bit 1);
+    // not where this is only walk_vertex_fast's fallback, whose registers
+    // would count for the whole kernel.
+    template <bool UNROLL = true>
+    __device__ __forceinline__ void sample(double en, double ex, double c0, double c1, double c2,
+                                           float (&cv)[8][NFP], int mval)
+    {
         __builtin_amdgcn_sched_barrier(0);
         // dt = (exit_t - enter_t) / n_samples, as a product with 1/n_samples.
         const double dt = (ex - en) * inv_ns;
@@ -765,8 +814,8 @@ struct VRSampler {
         float dp[3], ds[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            const int ci = (i == 0) ? c0 : ((i == 1) ? c1 : c2);
-            dp[i] = (float)(__builtin_fma(tt, pa[i], pb[i]) - (double)ci);
+            const double ci = (i == 0) ? c0 : ((i == 1) ? c1 : c2);
+            dp[i] = (float)(__builtin_fma(tt, pa[i], pb[i]) - ci);
             ds[i] = paf[i] * dtf;
         }
         // The positions are formed before the corner values are first used.
@@ -777,6 +826,7 @@ struct VRSampler {
             for (int f = 0; f < NFP; f++) asm volatile("" : "+v"(cv[q][f]));
         if (mval != 1) return;
         if (REC) rec->samples += n_samples;
+        constexpr int NS = (UNROLL && (MODE & 2)) ? 10 : 0;
         float k[NFP][4];
 #pragma unroll
         for (int f = 0; f < NFP; f++) {
@@ -784,7 +834,10 @@ struct VRSampler {
                                  cv[4][f], cv[5][f], cv[6][f], cv[7][f]};
             trilinear_cubic(cf, dp, ds, k[f]);
         }
-        if constexpr ((MODE & 1) != 0) {
+        if constexpr ((MODE & 32) != 0) {
+            ctf_visit_grey<NS>(*tf, lt, k[0], dt, n_samples, st);
+            return;
+        } else if constexpr ((MODE & 1) != 0) {
             float kq[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -796,16 +849,10 @@ struct VRSampler {
             // The bin coordinate u = v idbin + qc1 of the value's cubic.
             const float ku[4] = {__builtin_fmaf(kq[0], tf->idbin, tf->qc1), kq[1] * tf->idbin,
                                  kq[2] * tf->idbin, kq[3] * tf->idbin};
-            if (MODE & 2)
-                ctf_samples<10>(ku, dt, 10);
-            else
-                ctf_samples<0>(ku, dt, n_samples);
+            ctf_visit<NS>(*tf, lt, ku, (float)dt, n_samples, st);
             return;
         }
-        if (MODE & 2)
-            samples<10>(k, dt, 10);
-        else
-            samples<0>(k, dt, n_samples);
+        samples<NS>(k, dt, n_samples);
     }
 };
 
@@ -1051,6 +1098,102 @@ struct IProjSampler {
         }
     }
 };
+
+// walk_loop for a sampler of one vertex-centred field (S::sample; volume
+// renders with grey opacity), under
+// walk_vr_ctf_fast's conditions (walk_init left every walking lane inside
+// the brick, vertex blocks below 2^32 bytes, strides of 24 bits): no bounds
+// test per visit, the corners through a buffer resource at a 32-bit offset
+// summed over axes, cell indices also kept as doubles (stepped, exact) for
+// the sample positions, minima by one instruction, the axis step as nested
+// branches.  The sampler's arithmetic, and so every value, is that of
+// walk_loop.  SHARED: all rays have one direction (steps and increments are
+// scalar).
+template <bool SHARED, class S>
+__device__ __forceinline__ void walk_vertex_fast(Walk &w, double max_t, S &smp, __amdgpu_buffer_rsrc_t rsrc,
+                                                 unsigned K0, unsigned K1, const uint8_t *mask)
+{
+    double t0 = w.tmax[0], t1 = w.tmax[1], t2 = w.tmax[2];
+    int c0 = w.cur[0], c1 = w.cur[1], c2 = w.cur[2];
+    double en = w.enter_t;
+    const int st0 = SHARED ? uni(w.step[0]) : w.step[0], st1 = SHARED ? uni(w.step[1]) : w.step[1],
+              st2 = SHARED ? uni(w.step[2]) : w.step[2];
+    const double td0 = SHARED ? uni_d(w.tdelta[0]) : w.tdelta[0], td1 = SHARED ? uni_d(w.tdelta[1]) : w.tdelta[1],
+                 td2 = SHARED ? uni_d(w.tdelta[2]) : w.tdelta[2];
+    K0 = (unsigned)uni((int)K0);
+    K1 = (unsigned)uni((int)K1);
+    const unsigned D0 = (unsigned)smp.b.d0, D1 = (unsigned)smp.b.d1, D2 = (unsigned)smp.b.d2;
+    double f0 = (double)c0, f1 = (double)c1, f2 = (double)c2;
+    while (true) {
+        const bool a01 = t0 < t1;
+        const double m = min_f64(t0, t1);
+        const bool bm = m < t2;
+        const double tm = min_f64(m, t2);
+        const bool ge = tm >= max_t;
+        const double ex = min_f64(tm, max_t);
+        const unsigned o = __umul24((unsigned)c0 >> 2, K0) +
+                           (__umul24((unsigned)c1 >> 2, K1) +
+                            (__umul24((unsigned)c2 >> 2, VK2) +
+                             (__umul24((unsigned)c0, VW0) + (__umul24((unsigned)c1, VW1) + ((unsigned)c2 << 2)))));
+        int mval = 1;
+        if (mask != nullptr) mval = mask[(int)__umul24(__umul24(c0, D1) + c1, D2) + c2];
+        float cv[8][1];
+        {
+            float two[2];
+            BufLoad<2>::get(rsrc, o, two);
+            cv[0][0] = two[0], cv[1][0] = two[1];
+            BufLoad<2>::get(rsrc, o + 4u * vcorner(0, 1, 0), two);
+            cv[2][0] = two[0], cv[3][0] = two[1];
+            BufLoad<2>::get(rsrc, o + 4u * vcorner(1, 0, 0), two);
+            cv[4][0] = two[0], cv[5][0] = two[1];
+            BufLoad<2>::get(rsrc, o + 4u * vcorner(1, 1, 0), two);
+            cv[6][0] = two[0], cv[7][0] = two[1];
+        }
+        smp.sample(en, ex, f0, f1, f2, cv, mval);
+        bool out;
+        if (bm) {
+            if (a01) {
+                asm volatile("");
+                c0 += st0;
+                t0 += td0;
+                f0 = (double)c0;
+                out = (unsigned)c0 >= D0;
+            } else {
+                asm volatile("");
+                c1 += st1;
+                t1 += td1;
+                f1 = (double)c1;
+                out = (unsigned)c1 >= D1;
+            }
+        } else {
+            asm volatile("");
+            c2 += st2;
+            t2 += td2;
+            f2 = (double)c2;
+            out = (unsigned)c2 >= D2;
+        }
+        en = tm;
+        if (out || ge) break;
+    }
+}
+
+// The buffer resource and strides of a vertex brick for the fast walks, and
+// whether it and the wave's walking lanes meet their conditions
+// (walk_vr_ctf_fast).
+struct VertexFast {
+    bool ok;
+    unsigned bytes, k0, k1;
+};
+__device__ __forceinline__ VertexFast vertex_fast(const BrickReg &b, const Walk &w)
+{
+    const uint64_t bytes = (uint64_t)vblocks(b.d0) * (unsigned)b.vnbj * (unsigned)b.vnbk * (VBP * 4u);
+    const uint64_t k0 = vk0_bytes((unsigned)b.vnbj, (unsigned)b.vnbk);
+    const uint64_t k1 = vk1_bytes((unsigned)b.vnbk);
+    const bool inside = (unsigned)w.cur[0] < (unsigned)b.d0 && (unsigned)w.cur[1] < (unsigned)b.d1 &&
+                        (unsigned)w.cur[2] < (unsigned)b.d2;
+    return {bytes < (1ull << 32) && k0 < (1u << 24) && k1 < (1u << 24) && __all(inside), (unsigned)bytes,
+            (unsigned)k0, (unsigned)k1};
+}
 
 // LightSourceRenderSampler.sample (image_samplers.pyx:548-590) with
 // FIT_eval_transfer_with_light (field_interpolation_tables.pxd:115-143): per
@@ -1367,20 +1510,16 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
                 }
                 s.rec = &rec;
                 bool fastw = false;
-                if constexpr (!REC && NFP == 1 && (MODE & 1) != 0 && !PP) {
-                    // the fast walk's conditions (walk_vr_ctf_fast)
-                    const uint64_t bytes = (uint64_t)vblocks(s.b.d0) * (unsigned)s.b.vnbj *
-                                           (unsigned)s.b.vnbk * (VBP * 4u);
-                    const uint64_t k0 = vk0_bytes((unsigned)s.b.vnbj, (unsigned)s.b.vnbk);
-                    const bool inside = (unsigned)w.cur[0] < (unsigned)s.b.d0 &&
-                                        (unsigned)w.cur[1] < (unsigned)s.b.d1 &&
-                                        (unsigned)w.cur[2] < (unsigned)s.b.d2;
-                    const uint64_t k1 = vk1_bytes((unsigned)s.b.vnbk);
-                    if (bytes < (1ull << 32) && k0 < (1u << 24) && k1 < (1u << 24) && __all(inside)) {
-                        walk_vr_ctf_fast<(MODE & 2) ? 10 : 0, (MODE & 16) != 0>(
-                            w, max_t, s.b, brick_rsrc(s.data, (unsigned)bytes), (unsigned)k0,
-                            (unsigned)k1, s.mask, s.pa, s.pb, tfc, lt,
-                            s.inv_ns, s.n_samples, s.st, wbuf);
+                if constexpr (!REC && NFP == 1 && (MODE & 1) != 0 && ((MODE & 32) != 0 || !PP)) {
+                    const VertexFast vf = vertex_fast(s.b, w);
+                    if (vf.ok) {
+                        const __amdgpu_buffer_rsrc_t rs = brick_rsrc(s.data, vf.bytes);
+                        if constexpr ((MODE & 32) == 0)
+                            walk_vr_ctf_fast<(MODE & 2) ? 10 : 0, (MODE & 16) != 0>(
+                                w, max_t, s.b, rs, vf.k0, vf.k1, s.mask, s.pa, s.pb, tfc, lt, s.inv_ns, s.n_samples,
+                                s.st, wbuf);
+                        else
+                            walk_vertex_fast<!PP>(w, max_t, s, rs, vf.k0, vf.k1, s.mask);
                         fastw = true;
                     }
                 }
@@ -1485,13 +1624,18 @@ constexpr int QCOUNTERS = QSPLIT * QSTRIDE;  // words of counters per launch
 //   with the fast walk 2.3 % faster than 5 waves and within 0.5 % of 7;
 //   before it, 0.8 % faster than 5 waves (95 VGPRs, no spill), 2.5 %
 //   faster than 4, and 7 waves (72 VGPRs, 68-byte spill) 0.5 % slower;
+// - the same with grey opacity: 4 (128 VGPRs); 5 and 6 waves were 0 to 9 %
+//   slower;
 // - projection, one field, no record: 3.6 % faster than the 5 waves its
 //   90 VGPRs give.
 template <int KIND, int NFP, bool REC, int MODE>
 struct MinWaves {
-    static constexpr int value = (KIND == 1 && NFP == 1 && !REC && (MODE == 1 || MODE == 3 || MODE == 19)) ? 6
-                                 : (KIND == 0 && NFP == 1 && !REC)                          ? 6
-                                                                                             : 1;
+    static constexpr bool one = NFP == 1 && !REC;
+    static constexpr int value = !one                                                     ? 1
+                                 : (KIND == 1 && (MODE == 1 || MODE == 3 || MODE == 19)) ? 6
+                                 : (KIND == 1 && (MODE & 32) != 0)                       ? 4
+                                 : (KIND == 0)                                           ? 6
+                                                                                         : 1;
 };
 
 template <int KIND, int NFP, bool REC, int MODE>

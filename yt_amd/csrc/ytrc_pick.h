@@ -13,7 +13,8 @@ typedef void (*kfn_t)(const DImg *, int);
 // Each returns the variant for (nfp, rec, mode) within its unit's family,
 // or nullptr.  Families: projection, interpolated projection and light-source
 // rendering (modes 0, 8); volume rendering modes
-// 0-1, 2-3, 4-7 (early ray termination), 8-11 (per-pixel lens).
+// 0-1, 2-3, 4-7 (early ray termination), 8-11 (per-pixel lens), 33, 35, 41
+// and 43 (grey opacity).
 pfn_t pick_persist_proj(int nfp, bool rec, int mode);
 kfn_t pick_kernel_proj(int nfp, bool rec, int mode);
 pfn_t pick_persist_iproj(int nfp, bool rec, int mode);
@@ -28,5 +29,7 @@ pfn_t pick_persist_vr_c(int nfp, bool rec, int mode);
 kfn_t pick_kernel_vr_c(int nfp, bool rec, int mode);
 pfn_t pick_persist_vr_d(int nfp, bool rec, int mode);
 kfn_t pick_kernel_vr_d(int nfp, bool rec, int mode);
+pfn_t pick_persist_vr_e(int nfp, bool rec, int mode);
+kfn_t pick_kernel_vr_e(int nfp, bool rec, int mode);
 
 }  // namespace ytrc
