@@ -1392,10 +1392,10 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
         for (int c = 0; c < 3; c++) rgba0[c] = 1.0 - st[c];
     }
 
-    for (int kk = 0; kk < im.n_order; kk++) {
-        const int k = ert ? im.n_order - 1 - kk : kk;
+    // One brick of the order for every lane of the wave; true where the wave
+    // is done (early termination).
+    auto cast_brick = [&](int k) -> bool {
         const int4 e = im.ext[k];
-        if (e.y <= ti0 || e.x >= ti0 + th || e.w <= tj0 || e.z >= tj0 + tw) continue;
         bool go = active && vi >= e.x && vi < e.y && vj >= e.z && vj < e.w;
         const int bid = im.order[k];
         const DBrick &b = im.bricks[bid];
@@ -1549,8 +1549,30 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
         }
         if constexpr (ert) {
             const double tm = y_fmax(y_fmax(Tacc[0], Tacc[1]), y_fmax(Tacc[2], tfc.grey ? Tacc[3] : 0.0));
-            if (__all(!active || tm < ert_eps)) break;
+            if (__all(!active || tm < ert_eps)) return true;
         }
+        return false;
+    };
+    // The bricks whose extents meet the tile, in call order (reversed for
+    // early termination): each lane tests one of the next 64 bricks and the
+    // wave takes the hits from the ballot, one vector load for 64 extents
+    // instead of a scalar load, wait and branch for each.  On an AMR set a
+    // tile meets a few dozen of hundreds of bricks, and waves spent 69 % of
+    // their time waiting: 617 bricks at 700x500 took 0.385 ms, now 0.267
+    // (projection); 1672 bricks at 1024^2 2.23 ms, now 1.62 (volume render).
+    for (int base = 0; base < im.n_order; base += 64) {
+        const int kk = base + lane;
+        bool hit = false;
+        if (kk < im.n_order) {
+            const int4 e = im.ext[ert ? im.n_order - 1 - kk : kk];
+            hit = !(e.y <= ti0 || e.x >= ti0 + th || e.w <= tj0 || e.z >= tj0 + tw);
+        }
+        bool done = false;
+        for (uint64_t hits = __ballot(hit); hits != 0 && !done; hits &= hits - 1) {
+            const int k = base + __builtin_ctzll(hits);
+            done = cast_brick(ert ? im.n_order - 1 - k : k);
+        }
+        if (done) break;
     }
     if (!active) return;
     if (KIND == 0) {
