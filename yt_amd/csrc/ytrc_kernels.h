@@ -1649,11 +1649,15 @@ constexpr int QCOUNTERS = QSPLIT * QSTRIDE;  // words of counters per launch
 // - the same with grey opacity: 4 (128 VGPRs); 5 and 6 waves were 0 to 9 %
 //   slower;
 // - projection, one field, no record: 3.6 % faster than the 5 waves its
-//   90 VGPRs give.
+//   90 VGPRs give;
+// - projection, two fields (item x weight and weight): 4 (128 VGPRs) instead
+//   of the 3 its 131 give: 256^3 at 1024^2 0.416 -> 0.373 ms, 64 bricks of
+//   50^3 at 500x700 0.260 -> 0.229; 5 waves 0.377 and 0.248.
 template <int KIND, int NFP, bool REC, int MODE>
 struct MinWaves {
     static constexpr bool one = NFP == 1 && !REC;
-    static constexpr int value = !one                                                     ? 1
+    static constexpr int value = (KIND == 0 && NFP == 2 && !REC)                          ? 4
+                                 : !one                                                   ? 1
                                  : (KIND == 1 && (MODE == 1 || MODE == 3 || MODE == 19)) ? 6
                                  : (KIND == 1 && (MODE & 32) != 0)                       ? 4
                                  : (KIND == 0)                                           ? 6
