@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdint>
@@ -136,10 +137,41 @@ __global__ __launch_bounds__(256) void k_vertex_centre(VertexJob J, const T *__r
     }
 }
 
+// Clears the counters of n launches' queues.
 __global__ void k_zero_counters(unsigned int *c, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) c[i] = 0u;
+    if (i < n * QSPLIT) c[(size_t)i * QSTRIDE] = 0u;
+}
+
+// Moves staged data from pinned host memory to the device, one record per
+// blockIdx.x, STAGE_PARTS workgroups a record; and, for nv > 0 queues whose
+// item counts change from use to use, clears their counters and sets their
+// ranges' bounds to QSPLIT equal parts.  One launch in place of a copy each:
+// every copy of a few KB costs about 12 us of the host's time when it is
+// waited for, and the runtime runs it as a kernel of its own.
+struct StageRec {
+    const float4 *src;
+    float4 *dst;
+    uint64_t n;  // 16-byte units
+};
+struct QueueCounts {
+    int n[64];
+};
+constexpr int STAGE_PARTS = 8;
+__global__ __launch_bounds__(256) void k_stage(const StageRec *recs, unsigned int *c, QueueCounts q, int nv)
+{
+    const StageRec r = recs[blockIdx.x];
+    for (uint64_t i = blockIdx.y * 256u + threadIdx.x; i < r.n; i += STAGE_PARTS * 256u) r.dst[i] = r.src[i];
+    if (blockIdx.x != 0 || blockIdx.y != 0) return;
+    for (int i = threadIdx.x; i < nv * QSPLIT; i += 256) {
+        const int64_t n = q.n[i / QSPLIT];
+        const int part = i % QSPLIT;
+        unsigned int *w = c + (size_t)i * QSTRIDE;
+        w[0] = 0u;
+        w[QLO] = (unsigned int)(n * part / QSPLIT);
+        w[QHI] = (unsigned int)(n * (part + 1) / QSPLIT);
+    }
 }
 
 // Stores field f of one brick, uploaded in C order (src, or none for the
@@ -225,6 +257,112 @@ std::vector<int> tiles_z_order(int tiles0, int tiles1)
     return order;
 }
 
+// The estimated cost of each ray tile of one request, relative: the longest
+// chord of the rays at the tile's corners (plane-parallel lens) or centre
+// through the box around its bricks, plus 1/32 of that box's longest chord
+// for the tile itself.  Only the queue's order depends on it.
+std::vector<float> tile_costs(const ytrc_request &r, const DBrick *bricks, int tsh)
+{
+    const int th = 64 >> tsh, tw = 1 << tsh;
+    const int t0 = (r.nv[0] + th - 1) / th, t1 = (r.nv[1] + tw - 1) / tw;
+    double le[3] = {1e300, 1e300, 1e300}, re[3] = {-1e300, -1e300, -1e300};
+    for (int k = 0; k < r.n_order; k++)
+        for (int a = 0; a < 3; a++) {
+            le[a] = std::min(le[a], bricks[r.order[k]].le[a]);
+            re[a] = std::max(re[a], bricks[r.order[k]].re[a]);
+        }
+    // the part of a ray's [0, 1] inside the box
+    auto chord = [&](const double *pos, const double *iv, const double *dir) {
+        double a = 0.0, b = 1.0;
+        for (int i = 0; i < 3; i++) {
+            if (dir[i] == 0.0) {
+                if (pos[i] < le[i] || pos[i] > re[i]) return 0.0f;
+                continue;
+            }
+            const double p = (le[i] - pos[i]) * iv[i], q = (re[i] - pos[i]) * iv[i];
+            a = std::max(a, std::min(p, q));
+            b = std::min(b, std::max(p, q));
+        }
+        return (float)std::max(0.0, b - a);
+    };
+    std::vector<float> cost((size_t)t0 * t1);
+    float most = 0.0f;
+    if (r.lens == YTRC_LENS_PER_PIXEL) {
+        for (int i = 0; i < t0; i++)
+            for (int j = 0; j < t1; j++) {
+                const size_t pix = (size_t)std::min(i * th + th / 2, r.nv[0] - 1) * r.nv[1] +
+                                   std::min(j * tw + tw / 2, r.nv[1] - 1);
+                const double *dir = r.pix_dir + 3 * pix;
+                const double iv[3] = {1.0 / dir[0], 1.0 / dir[1], 1.0 / dir[2]};
+                cost[(size_t)i * t1 + j] = chord(r.pix_pos + 3 * pix, iv, dir);
+            }
+    } else {
+        const double iv[3] = {1.0 / r.vp_dir[0], 1.0 / r.vp_dir[1], 1.0 / r.vp_dir[2]};
+        std::vector<float> at((size_t)(t0 + 1) * (t1 + 1));
+        for (int i = 0; i <= t0; i++)
+            for (int j = 0; j <= t1; j++) {
+                // ray_setup's origins, to within a pixel
+                const double px = r.width[0] * ((double)std::min(i * th, r.nv[0]) / r.nv[0] - 0.5);
+                const double py = r.width[1] * ((double)std::min(j * tw, r.nv[1]) / r.nv[1] - 0.5);
+                double pos[3];
+                for (int a = 0; a < 3; a++) pos[a] = r.vp_pos[a] * px + r.vp_pos[3 + a] * py + r.vp_pos[9 + a];
+                at[(size_t)i * (t1 + 1) + j] = chord(pos, iv, r.vp_dir);
+            }
+        for (int i = 0; i < t0; i++)
+            for (int j = 0; j < t1; j++) {
+                const float *p = &at[(size_t)i * (t1 + 1) + j], *q = p + t1 + 1;
+                cost[(size_t)i * t1 + j] = std::max(std::max(p[0], p[1]), std::max(q[0], q[1]));
+            }
+    }
+    for (float c : cost) most = std::max(most, c);
+    for (float &c : cost) c += most > 0.0f ? most * (1.0f / 32.0f) : 1.0f;
+    return cost;
+}
+
+// The tiles 0 .. n - 1 of one image, in the order seq (or their own where it
+// is empty), cut into QSPLIT consecutive runs of about equal cost:
+// cut[0 .. QSPLIT].
+void equal_cost_runs(const std::vector<float> &cost, const std::vector<int> &seq, int cut[QSPLIT + 1])
+{
+    const int n = (int)cost.size();
+    double total = 0.0, sum = 0.0;
+    for (float c : cost) total += c;
+    int r = 1;
+    cut[0] = 0;
+    for (int t = 0; t < n && r < QSPLIT; t++) {
+        sum += cost[(size_t)(seq.empty() ? t : seq[(size_t)t])];
+        while (r < QSPLIT && sum * QSPLIT >= total * r) cut[r++] = t + 1;
+    }
+    while (r <= QSPLIT) cut[r++] = n;
+    cut[QSPLIT] = n;
+}
+
+// Sets the ranges' bounds in a launch's queue (host copy).
+void set_bounds(unsigned int *queue, const int cut[QSPLIT + 1])
+{
+    for (int r = 0; r < QSPLIT; r++) {
+        queue[r * QSTRIDE + QLO] = (unsigned int)cut[r];
+        queue[r * QSTRIDE + QHI] = (unsigned int)cut[r + 1];
+    }
+}
+
+// The step (0 .. 15) of a tile's cost in the costly-first order.
+int cost_step(float cost, float most) { return std::min(15, (int)(16.0f * cost / most)); }
+
+// Whether a launch of n single-tile items takes its costly tiles first.  It
+// evens out the SIMDs where few items follow the first ones; with more of
+// them the queue does, and the Z order keeps lines in L2.  Measured, kernel
+// time in launch order -> costly first: 256^3 volume render at 800x600 (1.2
+// items per slot) 1.02 -> 0.88 ms, 192^3 grey at 512^2 (0.7) 1.01 -> 0.87,
+// perspective 501x333 (0.4) 0.435 -> 0.413, 1672-brick render at 1024^2 (2.7)
+// 1.55 -> 1.55; projections, held by memory, 64 bricks at 500x700 (0.9) 0.224
+// -> 0.205, but 256^3 at 1024^2 (2.7) 0.379 -> 0.391.
+bool few_items(int n_cu, int kind, int64_t n)
+{
+    const int64_t slots = (int64_t)n_cu * 24;  // at 6 waves per SIMD
+    return n < (kind == YTRC_PROJECTION ? slots : 4 * slots);
+}
+
 // Words of LDS per wave that a persistent launch gives after its tables
 // (k_persist's wave_words): the vertex-block buffer with mode bit 4, a
 // projection's table of offset terms (walk_projection_fast).
@@ -307,6 +445,8 @@ struct Dataset {
 
 }  // namespace
 
+constexpr size_t PIN_BYTES = 2u << 20;
+
 struct ytrc_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -318,6 +458,7 @@ struct ytrc_ctx {
     int n_cu = 0;
     size_t max_lds = 64 * 1024;  // LDS bytes one workgroup may allocate
     std::string name;            // marketing name and ISA of the device
+    char *pin = nullptr;         // PIN_BYTES of pinned host memory (staging of ytrc_render_noalloc)
     char *scratch = nullptr;     // this device's `scratch` array (ytrc_render_noalloc)
     std::mutex *scratch_mu = nullptr;  // serialises the calls that share it
     std::map<int, Dataset> datasets;
@@ -674,10 +815,14 @@ int ytrc_ctx_create(int32_t device, uint64_t budget_bytes, ytrc_ctx **out)
         delete c;
         return fail(YTRC_EDEVICE, std::string("ytrc_ctx_create: second stream: ") + hipGetErrorString(e));
     }
-    if (scratch_setup(c) != YTRC_OK) {
+    int rc = scratch_setup(c);
+    if (rc == YTRC_OK && (e = hipHostMalloc((void **)&c->pin, PIN_BYTES, hipHostMallocDefault)) != hipSuccess)
+        rc = fail(YTRC_EDEVICE, std::string("ytrc_ctx_create: pinned staging: ") + hipGetErrorString(e));
+    if (rc != YTRC_OK) {
+        hipStreamDestroy(c->stream2);
         hipStreamDestroy(c->stream);
         delete c;
-        return YTRC_EDEVICE;
+        return rc;
     }
     *out = c;
     return YTRC_OK;
@@ -694,6 +839,7 @@ void ytrc_ctx_destroy(ytrc_ctx *ctx)
         hipFree(kv.second.d_pool);
         if (kv.second.d_masks) hipFree(kv.second.d_masks);
     }
+    if (ctx->pin) hipHostFree(ctx->pin);
     hipStreamDestroy(ctx->stream2);
     hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -961,9 +1107,16 @@ struct PrepReq {
     std::vector<float4> tft;
     size_t o_order = 0, o_ext = 0, o_zbuf = 0, o_init = 0, o_out = 0;
     size_t o_rv = 0, o_rh = 0, o_rs = 0, o_tf = 0, o_ppos = 0, o_pdir = 0;
-    size_t bytes = 0;
+    size_t up = 0;     // [0, up) is uploaded from a host copy (stage_request)
+    size_t bytes = 0;  // inputs, then outputs
+    bool inl = false;  // the per-pixel inputs are part of [0, up)
+    bool zbuf = false;  // a z-buffer that can end a ray
     int tsh = TILE_SHIFT_DEFAULT;
 };
+
+// Per-pixel inputs up to this many bytes travel with the request's host
+// copy; larger ones are copied from the caller's arrays directly.
+constexpr size_t INLINE_PIXELS = 256u << 10;
 
 // An upper bound of the t-interval of any ray of the request in one cell.
 double longest_cell_interval(const ytrc_request &r, const Dataset &ds, bool per_pixel)
@@ -1282,10 +1435,26 @@ int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, P
     off = align_up(off + sizeof(int32_t) * std::max(1, r.n_order), 256);
     P.o_ext = off;
     off = align_up(off + sizeof(int4) * P.ext.size(), 256);
+    P.o_tf = off;
+    if (has_tf(r.kind)) off = align_up(off + sizeof(DTF), 256);
+    P.up = off;
     P.o_zbuf = off;
     if (r.zbuffer) off = align_up(off + sizeof(double) * q.npix, 256);
     P.o_init = off;
     if (r.image_in && !additive_kind(r.kind)) off = align_up(off + sizeof(float) * 4 * q.npix, 256);
+    P.o_ppos = P.o_pdir = off;
+    if (pp) {
+        P.o_ppos = off;
+        off = align_up(off + sizeof(double) * 3 * q.npix, 256);
+        P.o_pdir = off;
+        off = align_up(off + sizeof(double) * 3 * q.npix, 256);
+    }
+    P.inl = off - P.up <= INLINE_PIXELS;
+    if (P.inl) P.up = off;
+    // max_t is the z value clamped to [0, 1]: at 1 everywhere it ends no ray
+    // (a NaN counts as 0 there).
+    if (r.zbuffer)
+        for (int64_t p = 0; p < q.npix && !P.zbuf; p++) P.zbuf = !(r.zbuffer[p] >= 1.0);
     P.o_out = off;
     off = align_up(off + sizeof(float) * std::max(4, q.nch_out) * q.npix, 256);
     P.o_rv = P.o_rh = P.o_rs = off;
@@ -1297,24 +1466,16 @@ int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, P
         P.o_rs = off;
         off = align_up(off + 8 * q.npix, 256);
     }
-    P.o_tf = off;
-    if (has_tf(r.kind)) off = align_up(off + sizeof(DTF), 256);
-    P.o_ppos = P.o_pdir = off;
-    if (pp) {
-        P.o_ppos = off;
-        off = align_up(off + sizeof(double) * 3 * q.npix, 256);
-        P.o_pdir = off;
-        off = align_up(off + sizeof(double) * 3 * q.npix, 256);
-    }
     P.bytes = off;
     return YTRC_OK;
 }
 
-// Copies a prepared request into its device region `A` and fills its
+// Writes a prepared request's inputs to `H`, the host copy of bytes [0, P.up)
+// of its device region `A` (the caller moves them there before a launch reads
+// them), copies large per-pixel inputs to the region directly, and fills its
 // device descriptor.  `tf_table` is the device address of its (deduplicated)
 // transfer-function table, at float4 offset `tf_slot` of the launch's table.
-int stage_request(ytrc_ctx *ctx, PrepReq &P, char *A, const float4 *tf_table, int tf_slot, DImg &d,
-                  std::vector<float> &stage)
+int stage_request(ytrc_ctx *ctx, PrepReq &P, char *H, char *A, const float4 *tf_table, int tf_slot, DImg &d)
 {
     const ytrc_request &r = P.q.r;
     const ReqHost &q = P.q;
@@ -1329,7 +1490,7 @@ int stage_request(ytrc_ctx *ctx, PrepReq &P, char *A, const float4 *tf_table, in
     d.masks = ds.d_masks;
     d.order = (const int32_t *)(A + P.o_order);
     d.ext = (const int4 *)(A + P.o_ext);
-    d.zbuf = r.zbuffer ? (const double *)(A + P.o_zbuf) : nullptr;
+    d.zbuf = P.zbuf ? (const double *)(A + P.o_zbuf) : nullptr;
     const bool init_dev = r.image_in != nullptr && !additive_kind(r.kind);
     d.init = init_dev ? (const float *)(A + P.o_init) : nullptr;
     d.out = (float *)(A + P.o_out);
@@ -1354,28 +1515,32 @@ int stage_request(ytrc_ctx *ctx, PrepReq &P, char *A, const float4 *tf_table, in
     d.inv_ns = r.n_samples > 0 ? 1.0 / (double)r.n_samples : 0.0;
     d.tform = q.tform;
     if (r.n_order > 0) {
-        HIPCHK(hipMemcpy(A + P.o_order, r.order, sizeof(int32_t) * r.n_order, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(A + P.o_ext, P.ext.data(), sizeof(int4) * r.n_order, hipMemcpyHostToDevice));
+        memcpy(H + P.o_order, r.order, sizeof(int32_t) * r.n_order);
+        memcpy(H + P.o_ext, P.ext.data(), sizeof(int4) * r.n_order);
     }
-    if (r.zbuffer)
-        HIPCHK(hipMemcpy(A + P.o_zbuf, r.zbuffer, sizeof(double) * q.npix, hipMemcpyHostToDevice));
+    auto pixels = [&](size_t at, const void *src, size_t bytes) {
+        if (!P.inl) return hipMemcpy(A + at, src, bytes, hipMemcpyHostToDevice);
+        memcpy(H + at, src, bytes);
+        return hipSuccess;
+    };
+    if (P.zbuf) HIPCHK(pixels(P.o_zbuf, r.zbuffer, sizeof(double) * q.npix));
     if (r.lens == YTRC_LENS_PER_PIXEL) {
         d.pix_pos = (const double *)(A + P.o_ppos);
         d.pix_dir = (const double *)(A + P.o_pdir);
-        HIPCHK(hipMemcpy(A + P.o_ppos, r.pix_pos, sizeof(double) * 3 * q.npix, hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(A + P.o_pdir, r.pix_dir, sizeof(double) * 3 * q.npix, hipMemcpyHostToDevice));
+        HIPCHK(pixels(P.o_ppos, r.pix_pos, sizeof(double) * 3 * q.npix));
+        HIPCHK(pixels(P.o_pdir, r.pix_dir, sizeof(double) * 3 * q.npix));
     }
     if (init_dev) {
-        stage.resize((size_t)q.npix * 4);
+        std::vector<float> stage((size_t)q.npix * 4);
         for (int64_t p = 0; p < q.npix; p++)
             for (int c = 0; c < 4; c++) stage[(size_t)c * q.npix + p] = (float)r.image_in[p * 4 + c];
-        HIPCHK(hipMemcpy(A + P.o_init, stage.data(), sizeof(float) * 4 * q.npix, hipMemcpyHostToDevice));
+        HIPCHK(pixels(P.o_init, stage.data(), sizeof(float) * 4 * q.npix));
     }
     if (has_tf(r.kind)) {
         DTF T = P.T;
         T.table = tf_table + tf_slot;
         d.tf_slot = tf_slot;
-        HIPCHK(hipMemcpy(A + P.o_tf, &T, sizeof(DTF), hipMemcpyHostToDevice));
+        memcpy(H + P.o_tf, &T, sizeof(DTF));
     }
     return YTRC_OK;
 }
@@ -1548,21 +1713,31 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     }
     const size_t tfall_off = off;
     off = align_up(off + sizeof(float4) * std::max<size_t>(1, tf_all.size()), 256);
-    // Each image's tiles are cut into QSPLIT contiguous chunks and chunk r
-    // goes to queue range r (the range one XCD drains first), so every XCD
-    // renders a compact part of every image; within a range the images
-    // advance together (items ordered by the fraction of their chunk done,
+    // Each image's tiles are cut into QSPLIT contiguous runs of equal
+    // estimated cost and run r goes to queue range r (the range one XCD
+    // drains first), so every XCD renders a compact part of every image and
+    // has the same work: with runs of equal length, the XCDs of an image's
+    // middle had up to twice the work of those of its rim, all of it already
+    // in flight when the others ran dry (256^3 in an 800x600 view: 2.1 of 6
+    // waves per SIMD resident on average).  Within a range the images advance
+    // together (items ordered by the fraction of their run's cost done,
     // larger images first on ties).  Waves of small images, whose rays are
     // sparser than the cells and wait on memory, then run beside waves of
     // large images, which keep the VALUs busy: 5-6 % faster than running
     // the images one after another, larger first.
+    // A launch with few items per wave slot (few_items) takes each range's
+    // costly tiles first instead, in 16 steps of cost and Z order within a
+    // step: nearly all its items are in flight at once, and waves start
+    // SIMD after SIMD, so each SIMD gets its share of every step.
     std::vector<std::vector<int2>> gitems;
+    std::vector<std::array<int, QSPLIT + 1>> gbounds;
     std::vector<size_t> gitems_off;
     for (size_t L = 0; L < plans.size(); L++) {
         std::vector<int> ids = plans[L].ids;
         std::stable_sort(ids.begin(), ids.end(),
                          [&](int a, int b) { return P[a].q.ntiles > P[b].q.ntiles; });
         std::vector<int2> items;
+        std::array<int, QSPLIT + 1> bounds;
         struct Key {
             double frac;
             int ord;
@@ -1574,25 +1749,38 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         // kernel 1.2 % faster, the volume-render kernel alone 0.4 % slower,
         // the two launches together 0.7 % faster than in row order.
         const bool z = per_item == 1;
+        int64_t ntiles = 0;
+        for (int i : ids) ntiles += P[i].q.ntiles;
+        const bool costly_first = z && few_items(ctx->n_cu, std::get<0>(plans[L].variant), ntiles);
         std::vector<std::vector<int>> zord(ids.size());
-        if (z)
-            for (size_t o = 0; o < ids.size(); o++) {
-                const PrepReq &Q = P[ids[o]];
-                const int th = 64 >> Q.tsh, tw = 1 << Q.tsh;
-                zord[o] = tiles_z_order((Q.q.r.nv[0] + th - 1) / th, (Q.q.r.nv[1] + tw - 1) / tw);
-            }
+        std::vector<std::vector<float>> cost(ids.size());
+        std::vector<float> most(ids.size());
+        std::vector<std::array<int, QSPLIT + 1>> cut(ids.size());
+        for (size_t o = 0; o < ids.size(); o++) {
+            const PrepReq &Q = P[ids[o]];
+            const int th = 64 >> Q.tsh, tw = 1 << Q.tsh;
+            if (z) zord[o] = tiles_z_order((Q.q.r.nv[0] + th - 1) / th, (Q.q.r.nv[1] + tw - 1) / tw);
+            cost[o] = tile_costs(reqs[ids[o]], ctx->datasets[reqs[ids[o]].ds_id].h_bricks.data(), Q.tsh);
+            most[o] = *std::max_element(cost[o].begin(), cost[o].end());
+            equal_cost_runs(cost[o], zord[o], cut[o].data());
+        }
         for (int r = 0; r < QSPLIT; r++) {
+            bounds[(size_t)r] = (int)items.size();
             std::vector<Key> ks;
             for (size_t o = 0; o < ids.size(); o++) {
                 const int i = ids[o];
-                const int T = P[i].q.ntiles;
-                const int t0 = (int)((int64_t)r * T / QSPLIT), t1 = (int)((int64_t)(r + 1) * T / QSPLIT);
+                const int t0 = cut[o][(size_t)r], t1 = cut[o][(size_t)r + 1];
+                double total = 0.0, done = 0.0;
+                for (int t = t0; t < t1; t++) total += cost[o][(size_t)(z ? zord[o][(size_t)t] : t)];
                 // an item: up to per_item consecutive tiles, the count in
                 // the top 8 bits of its tile field
                 for (int t = t0; t < t1; t += per_item) {
                     const int cnt = std::min(per_item, t1 - t);
                     const int tile = z ? zord[o][(size_t)t] : t;
-                    ks.push_back({(double)(t - t0) / (double)(t1 - t0), (int)o, make_int2(i, tile | (cnt << 24))});
+                    const double key = costly_first ? (double)-cost_step(cost[o][(size_t)tile], most[o])
+                                                    : done / total;
+                    ks.push_back({key, (int)o, make_int2(i, tile | (cnt << 24))});
+                    for (int q = 0; q < cnt; q++) done += cost[o][(size_t)(z ? zord[o][(size_t)(t + q)] : t + q)];
                 }
             }
             std::stable_sort(ks.begin(), ks.end(), [](const Key &a, const Key &b) {
@@ -1600,6 +1788,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
             });
             for (const Key &k : ks) items.push_back(k.item);
         }
+        bounds[QSPLIT] = (int)items.size();
         PGroup g;
         g.kind = std::get<0>(plans[L].variant);
         g.nfp = std::get<1>(plans[L].variant);
@@ -1627,6 +1816,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         gitems_off.push_back(off);
         off = align_up(off + sizeof(int2) * std::max<size_t>(1, items.size()), 256);
         gitems.push_back(std::move(items));
+        gbounds.push_back(bounds);
     }
     const size_t counters_off = off;
     off = align_up(off + sizeof(unsigned int) * QCOUNTERS * std::max<size_t>(1, B->groups.size()), 256);
@@ -1639,30 +1829,6 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     B->arena_bytes = off;
     ctx->used += off;
     char *A = B->arena;
-    std::vector<float> stage;
-    for (int i = 0; i < n_req; i++) {
-        const int rc = stage_request(ctx, P[i], A + base[i], (const float4 *)(A + tfall_off), slot[i],
-                                     B->h_imgs[i], stage);
-        if (rc != YTRC_OK) return bad(rc, g_err);
-        // the persistent kernels read the table from their launch's block
-        B->h_imgs[i].tf_slot = rel_slot[i];
-    }
-    B->tf_all = (const float4 *)(A + tfall_off);
-    B->tf_bins = (int)tf_all.size();
-    if (!tf_all.empty()) {
-        e = hipMemcpy(A + tfall_off, tf_all.data(), sizeof(float4) * tf_all.size(), hipMemcpyHostToDevice);
-        if (e != hipSuccess) return bad(YTRC_EDEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
-    }
-    for (size_t g = 0; g < B->groups.size(); g++) {
-        B->groups[g].items = (const int2 *)(A + gitems_off[g]);
-        if (!gitems[g].empty()) {
-            e = hipMemcpy(A + gitems_off[g], gitems[g].data(), sizeof(int2) * gitems[g].size(),
-                          hipMemcpyHostToDevice);
-            if (e != hipSuccess) return bad(YTRC_EDEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
-        }
-    }
-    B->counters = (unsigned int *)(A + counters_off);
-    B->d_imgs = (DImg *)(A + imgs_off);
     // The stop flag: fine-grained pinned host memory that the kernels read
     // at system scope once per tile.
     e = hipHostMalloc((void **)&B->h_stop, sizeof(int), hipHostMallocCoherent | hipHostMallocMapped);
@@ -1671,9 +1837,37 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     int *d_stop = nullptr;
     e = hipHostGetDevicePointer((void **)&d_stop, B->h_stop, 0);
     if (e != hipSuccess) return bad(YTRC_EDEVICE, std::string("hipHostGetDevicePointer: ") + hipGetErrorString(e));
-    for (int i = 0; i < n_req; i++) B->h_imgs[i].stop = d_stop;
-    e = hipMemcpy(B->d_imgs, B->h_imgs.data(), sizeof(DImg) * n_req, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return bad(YTRC_EDEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
+    auto put = [&](size_t at, const void *src, size_t bytes) {
+        return bytes ? hipMemcpy(A + at, src, bytes, hipMemcpyHostToDevice) : hipSuccess;
+    };
+    std::vector<char> host;
+    for (int i = 0; i < n_req; i++) {
+        host.assign(P[i].up, 0);
+        const int rc = stage_request(ctx, P[i], host.data(), A + base[i], (const float4 *)(A + tfall_off), slot[i],
+                                     B->h_imgs[i]);
+        if (rc != YTRC_OK) return bad(rc, g_err);
+        if ((e = put(base[i], host.data(), P[i].up)) != hipSuccess)
+            return bad(YTRC_EDEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
+        // the persistent kernels read the table from their launch's block
+        B->h_imgs[i].tf_slot = rel_slot[i];
+        B->h_imgs[i].stop = d_stop;
+    }
+    // The tables, items, queues and descriptors lie back to back: one copy.
+    host.assign(off - tfall_off, 0);
+    auto at = [&](size_t o) { return host.data() + (o - tfall_off); };
+    if (!tf_all.empty()) memcpy(at(tfall_off), tf_all.data(), sizeof(float4) * tf_all.size());
+    for (size_t g = 0; g < B->groups.size(); g++) {
+        B->groups[g].items = (const int2 *)(A + gitems_off[g]);
+        if (!gitems[g].empty()) memcpy(at(gitems_off[g]), gitems[g].data(), sizeof(int2) * gitems[g].size());
+        set_bounds((unsigned int *)at(counters_off) + QCOUNTERS * g, gbounds[g].data());
+    }
+    memcpy(at(imgs_off), B->h_imgs.data(), sizeof(DImg) * n_req);
+    if ((e = put(tfall_off, host.data(), host.size())) != hipSuccess)
+        return bad(YTRC_EDEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
+    B->tf_all = (const float4 *)(A + tfall_off);
+    B->tf_bins = (int)tf_all.size();
+    B->counters = (unsigned int *)(A + counters_off);
+    B->d_imgs = (DImg *)(A + imgs_off);
     if ((e = hipEventCreate(&B->ev0)) != hipSuccess || (e = hipEventCreate(&B->ev1)) != hipSuccess)
         return bad(YTRC_EDEVICE, std::string("hipEventCreate: ") + hipGetErrorString(e));
     if (batch_flags & YTRC_BATCH_PERSISTENT) {
@@ -1736,8 +1930,7 @@ namespace {
 int enqueue_persistent(ytrc_batch *b, hipStream_t s)
 {
     const int ng = (int)b->groups.size();
-    hipLaunchKernelGGL(k_zero_counters, dim3((ng * QCOUNTERS + 255) / 256), dim3(256), 0, s, b->counters,
-                       ng * QCOUNTERS);
+    hipLaunchKernelGGL(k_zero_counters, dim3((ng * QSPLIT + 255) / 256), dim3(256), 0, s, b->counters, ng);
     HIPCHK(hipGetLastError());
     const int threads = 64 * b->waves_per_group;
     // The launches run concurrently: the one with the most estimated work
@@ -1775,7 +1968,7 @@ int enqueue_persistent(ytrc_batch *b, hipStream_t s)
         g.grid = std::max(1, std::min(per_cu * b->ctx->n_cu,
                                       (g.n_items + b->waves_per_group - 1) / b->waves_per_group));
         hipLaunchKernelGGL(g.fn, dim3(g.grid), dim3(threads), lds, gs, (const DImg *)b->d_imgs,
-                           g.items, g.n_items, b->counters + (size_t)g.counter * QCOUNTERS, b->tf_all + g.tf_base,
+                           g.items, b->counters + (size_t)g.counter * QCOUNTERS, b->tf_all + g.tf_base,
                            g.tf_bins, ww);
         HIPCHK(hipGetLastError());
     }
@@ -1871,20 +2064,44 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
                                      " B of device staging, more than the " +
                                      std::to_string((size_t)YTRC_NOALLOC_SCRATCH_BYTES) +
                                      " B fixed array; use ytrc_batch_create");
+    // The host copy of what the device needs: the request's inputs and, from
+    // tf_off on, everything after its outputs.  In the context's pinned
+    // memory if it fits there (the mutexes are held until the call's stream
+    // is idle), moved by k_stage; otherwise copied.
     char *S = ctx->scratch;
+    const size_t rec_bytes = 256, tail = off - tf_off;
+    const bool pinned = rec_bytes + P.up + tail <= PIN_BYTES;
+    std::vector<char> pageable(pinned ? 0 : P.up + tail);
+    char *H = pinned ? ctx->pin + rec_bytes : pageable.data();
+    char *Ht = H + P.up;
     DImg d;
-    std::vector<float> stage;
-    rc = stage_request(ctx, P, S, (const float4 *)(S + tf_off), 0, d, stage);
+    rc = stage_request(ctx, P, H, S, (const float4 *)(S + tf_off), 0, d);
     if (rc != YTRC_OK) return rc;
-    if (!P.tft.empty())
-        HIPCHK(hipMemcpy(S + tf_off, P.tft.data(), sizeof(float4) * P.tft.size(), hipMemcpyHostToDevice));
-    // One request: the tiles in order (the QSPLIT queue ranges are its
-    // QSPLIT contiguous chunks, as in a persistent batch of this request).
-    std::vector<int2> items((size_t)P.q.ntiles);
-    for (int t = 0; t < P.q.ntiles; t++) items[(size_t)t] = make_int2(0, t);
-    if (!items.empty())
-        HIPCHK(hipMemcpy(S + items_off, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(S + img_off, &d, sizeof(DImg), hipMemcpyHostToDevice));
+    if (!P.tft.empty()) memcpy(Ht, P.tft.data(), sizeof(float4) * P.tft.size());
+    // One request: the tiles in row order, cut into QSPLIT runs of equal
+    // cost; with few of them, costly ones first within a run, as in a batch.
+    int2 *items = (int2 *)(Ht + (items_off - tf_off));
+    int cut[QSPLIT + 1];
+    {
+        const std::vector<float> cost = tile_costs(*req, ctx->datasets[req->ds_id].h_bricks.data(), P.tsh);
+        equal_cost_runs(cost, {}, cut);
+        if (few_items(ctx->n_cu, req->kind, P.q.ntiles)) {
+            const float most = *std::max_element(cost.begin(), cost.end());
+            for (int r = 0; r < QSPLIT; r++) {
+                int at[17] = {0};
+                for (int t = cut[r]; t < cut[r + 1]; t++) at[16 - cost_step(cost[(size_t)t], most)]++;
+                for (int q = 1; q < 17; q++) at[q] += at[q - 1];
+                for (int t = cut[r]; t < cut[r + 1]; t++)
+                    items[(size_t)(cut[r] + at[15 - cost_step(cost[(size_t)t], most)]++)] = make_int2(0, t);
+            }
+        } else {
+            for (int t = 0; t < P.q.ntiles; t++) items[(size_t)t] = make_int2(0, t);
+        }
+    }
+    unsigned int *queue = (unsigned int *)(Ht + (cnt_off - tf_off));
+    memset(queue, 0, sizeof(unsigned int) * QCOUNTERS);
+    set_bounds(queue, cut);
+    memcpy(Ht + (img_off - tf_off), &d, sizeof(DImg));
     const pfn_t fn = pick_persist(req->kind, P.q.nfp, false, P.q.mode);
     if (fn == nullptr) return fail(YTRC_ENOTIMPL, "ytrc_render_noalloc: no kernel for this request");
     const int wpg = 4, threads = 64 * wpg;
@@ -1894,15 +2111,23 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
         HIPCHK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipStream_t s = ctx->stream;
     unsigned int *counters = (unsigned int *)(S + cnt_off);
-    // the array keeps the previous call's counters: clear them
-    hipLaunchKernelGGL(k_zero_counters, dim3((QCOUNTERS + 255) / 256), dim3(256), 0, s, counters, QCOUNTERS);
-    HIPCHK(hipGetLastError());
+    if (pinned) {
+        StageRec *recs = (StageRec *)ctx->pin;
+        recs[0] = {(const float4 *)H, (float4 *)S, P.up / 16};
+        recs[1] = {(const float4 *)Ht, (float4 *)(S + tf_off), tail / 16};
+        hipLaunchKernelGGL(k_stage, dim3(2, STAGE_PARTS), dim3(256), 0, s, (const StageRec *)recs, nullptr,
+                           QueueCounts{}, 0);
+        HIPCHK(hipGetLastError());
+    } else {
+        HIPCHK(hipMemcpy(S, H, P.up, hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(S + tf_off, Ht, tail, hipMemcpyHostToDevice));
+    }
     if (P.q.ntiles > 0) {
         int nb = 0;
         HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, threads, lds));
         const int grid = std::max(1, std::min(std::max(1, nb) * ctx->n_cu, (P.q.ntiles + wpg - 1) / wpg));
         hipLaunchKernelGGL(fn, dim3(grid), dim3(threads), lds, s, (const DImg *)(S + img_off),
-                           (const int2 *)(S + items_off), P.q.ntiles, counters,
+                           (const int2 *)(S + items_off), counters,
                            (const float4 *)(S + tf_off), (int)P.tft.size(), ww);
         HIPCHK(hipGetLastError());
     }
@@ -2170,6 +2395,8 @@ struct SrvReq {
     int state = 0;  // 0 tiles pending, 1 all tiles launched, 2 done, 3 cancelled
     int tf_entry = -1;
     bool ds_ref = false;  // holds a reference on its dataset
+    std::vector<char> host;  // inputs not yet on the device: they go with its first chunk
+    bool staged = false;     // its inputs and descriptor are on the device, or launched to be
     std::chrono::steady_clock::time_point t_submit;
 };
 
@@ -2183,7 +2410,9 @@ struct TFEntry {
 struct SrvChunk {
     int64_t seq = -1;
     hipEvent_t done = nullptr;
+    hipEvent_t staged = nullptr;  // its k_stage
     int2 *h_items = nullptr;  // pinned
+    char *h_stage = nullptr;  // pinned: SRV_RECS records, then SRV_STAGE bytes of new requests' inputs
     int2 *d_items = nullptr;
     unsigned int *d_counters = nullptr;
     std::vector<int64_t> finishing;
@@ -2191,7 +2420,14 @@ struct SrvChunk {
 };
 
 constexpr int SRV_CHUNKS = 3;
+// One chunk's staging: records (one for the items, two per request that
+// starts in it) and input bytes.  A request that finds no room, or whose
+// inputs are larger than a quarter of it, is copied directly.
+constexpr int SRV_RECS = 129;
+constexpr size_t SRV_STAGE = 512u << 10;
+constexpr size_t SRV_STAGE_BYTES = SRV_STAGE + 256 * ((SRV_RECS * sizeof(StageRec) + 255) / 256);
 constexpr int SRV_MAX_VARIANTS = 64;  // distinct persistent kernels one server launches
+static_assert(sizeof(QueueCounts) / sizeof(int) == SRV_MAX_VARIANTS, "a count per variant");
 
 }  // namespace
 
@@ -2390,6 +2626,9 @@ int srv_pump(ytrc_server *S)
         // finished only once every chunk that holds its tiles has retired.
         hipStream_t s = (S->chunks_launched & 1) ? S->ctx->stream2 : s0;
         C.finishing.clear();
+        StageRec *recs = (StageRec *)C.h_stage;
+        char *sp = C.h_stage + (SRV_STAGE_BYTES - SRV_STAGE), *const send = C.h_stage + SRV_STAGE_BYTES;
+        int nrec = 1;  // recs[0]: the items
         const int nv = (int)S->vkeys.size();
         std::vector<std::vector<int2>> per(nv);
         int filled = 0;
@@ -2397,6 +2636,22 @@ int srv_pump(ytrc_server *S)
         for (int64_t id : srv_fill_order(S)) {
             if (filled >= S->chunk_tiles) break;
             SrvReq &R = S->reqs.at(id);
+            if (!R.staged) {
+                const size_t bytes = R.host.size() + sizeof(DImg);
+                if (nrec + 2 <= SRV_RECS && bytes <= (size_t)(send - sp) && R.host.size() <= SRV_STAGE / 4) {
+                    memcpy(sp, R.host.data(), R.host.size());
+                    memcpy(sp + R.host.size(), &R.d, sizeof(DImg));
+                    recs[nrec++] = {(const float4 *)sp, (float4 *)(S->arena + R.off), R.host.size() / 16};
+                    recs[nrec++] = {(const float4 *)(sp + R.host.size()), (float4 *)(S->d_slots + R.slot),
+                                    sizeof(DImg) / 16};
+                    sp += bytes;
+                } else {
+                    HIPCHK(hipMemcpy(S->arena + R.off, R.host.data(), R.host.size(), hipMemcpyHostToDevice));
+                    HIPCHK(hipMemcpy(S->d_slots + R.slot, &R.d, sizeof(DImg), hipMemcpyHostToDevice));
+                }
+                R.staged = true;
+                R.host = std::vector<char>();
+            }
             const int take = std::min(R.P.q.ntiles - R.next_tile, S->chunk_tiles - filled);
             for (int t = 0; t < take; t++) per[R.variant].push_back(make_int2(R.slot, R.next_tile + t));
             R.next_tile += take;
@@ -2419,10 +2674,16 @@ int srv_pump(ytrc_server *S)
             vcnt[v] = (int)per[v].size();
             for (auto &it : per[v]) C.h_items[n++] = it;
         }
-        HIPCHK(hipMemcpyAsync(C.d_items, C.h_items, sizeof(int2) * n, hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(k_zero_counters, dim3((SRV_MAX_VARIANTS * QCOUNTERS + 255) / 256), dim3(256), 0, s,
-                           C.d_counters, SRV_MAX_VARIANTS * QCOUNTERS);
+        // One launch moves the items and the new requests' inputs and sets up
+        // the queues.  The chunk before this one, on the other stream, may
+        // have staged a request whose other tiles are in this one.
+        recs[0] = {(const float4 *)C.h_items, (float4 *)C.d_items, (sizeof(int2) * (size_t)n + 15) / 16};
+        QueueCounts qc{};
+        for (int v = 0; v < nv; v++) qc.n[v] = vcnt[v];
+        for (int ci2 : S->inflight) HIPCHK(hipStreamWaitEvent(s, S->chunks[ci2].staged, 0));
+        hipLaunchKernelGGL(k_stage, dim3(nrec, STAGE_PARTS), dim3(256), 0, s, (const StageRec *)recs, C.d_counters, qc, nv);
         HIPCHK(hipGetLastError());
+        HIPCHK(hipEventRecord(C.staged, s));
         for (int v = 0; v < nv; v++) {
             if (vcnt[v] == 0) continue;
             const bool vr = has_tf(std::get<0>(S->vkeys[v]));
@@ -2433,7 +2694,7 @@ int srv_pump(ytrc_server *S)
             HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, S->vfns[v], 256, lds));
             const int grid = std::max(1, std::min(std::max(1, nb) * S->ctx->n_cu, (vcnt[v] + 3) / 4));
             hipLaunchKernelGGL(S->vfns[v], dim3(grid), dim3(256), lds, s, (const DImg *)S->d_slots,
-                               (const int2 *)(C.d_items + voff[v]), vcnt[v], C.d_counters + (size_t)v * QCOUNTERS,
+                               (const int2 *)(C.d_items + voff[v]), C.d_counters + (size_t)v * QCOUNTERS,
                                (const float4 *)S->d_tf, vr ? S->tf_hi : 0, ww);
             HIPCHK(hipGetLastError());
         }
@@ -2503,7 +2764,9 @@ int ytrc_server_create(ytrc_ctx *ctx, int32_t max_requests, uint64_t budget_byte
             if (c.h_items) hipHostFree(c.h_items);
             if (c.d_items) hipFree(c.d_items);
             if (c.d_counters) hipFree(c.d_counters);
+            if (c.h_stage) hipHostFree(c.h_stage);
             if (c.done) hipEventDestroy(c.done);
+            if (c.staged) hipEventDestroy(c.staged);
         }
         delete S;
         return fail(YTRC_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
@@ -2517,13 +2780,18 @@ int ytrc_server_create(ytrc_ctx *ctx, int32_t max_requests, uint64_t budget_byte
     e = hipMalloc(&S->d_tf, sizeof(float4) * S->tf_cap);
     if (e != hipSuccess) return bad(e, "hipMalloc(tf)");
     for (auto &c : S->chunks) {
-        e = hipHostMalloc(&c.h_items, sizeof(int2) * chunk_tiles, hipHostMallocDefault);
+        // (k_stage moves whole 16-byte units)
+        e = hipHostMalloc(&c.h_items, sizeof(int2) * (chunk_tiles + 1), hipHostMallocDefault);
         if (e != hipSuccess) return bad(e, "hipHostMalloc(items)");
-        e = hipMalloc(&c.d_items, sizeof(int2) * chunk_tiles);
+        e = hipHostMalloc((void **)&c.h_stage, SRV_STAGE_BYTES, hipHostMallocDefault);
+        if (e != hipSuccess) return bad(e, "hipHostMalloc(staging)");
+        e = hipMalloc(&c.d_items, sizeof(int2) * (chunk_tiles + 1));
         if (e != hipSuccess) return bad(e, "hipMalloc(items)");
         e = hipMalloc(&c.d_counters, sizeof(unsigned int) * SRV_MAX_VARIANTS * QCOUNTERS);
         if (e != hipSuccess) return bad(e, "hipMalloc(counters)");
         e = hipEventCreateWithFlags(&c.done, hipEventDisableTiming);
+        if (e != hipSuccess) return bad(e, "hipEventCreate");
+        e = hipEventCreateWithFlags(&c.staged, hipEventDisableTiming);
         if (e != hipSuccess) return bad(e, "hipEventCreate");
     }
     for (int i = max_requests - 1; i >= 0; i--) S->free_slots.push_back(i);
@@ -2579,12 +2847,8 @@ int ytrc_server_submit(ytrc_server *S, const ytrc_request *r, int64_t *id_out)
     }
     R.slot = S->free_slots.back();
     S->free_slots.pop_back();
-    std::vector<float> stage;
-    int rc = stage_request(S->ctx, R.P, S->arena + off, S->d_tf, tf_base, R.d, stage);
-    if (rc == YTRC_OK) {
-        hipError_t e = hipMemcpy(S->d_slots + R.slot, &R.d, sizeof(DImg), hipMemcpyHostToDevice);
-        if (e != hipSuccess) rc = fail(YTRC_EDEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
-    }
+    R.host.assign(R.P.up, 0);
+    int rc = stage_request(S->ctx, R.P, R.host.data(), S->arena + off, S->d_tf, tf_base, R.d);
     if (rc != YTRC_OK) {
         srv_release(S, R);
         return rc;
@@ -2779,9 +3043,11 @@ void ytrc_server_destroy(ytrc_server *S)
     hipFree(S->d_tf);
     for (auto &c : S->chunks) {
         hipHostFree(c.h_items);
+        hipHostFree(c.h_stage);
         hipFree(c.d_items);
         hipFree(c.d_counters);
         hipEventDestroy(c.done);
+        hipEventDestroy(c.staged);
     }
     {
         std::lock_guard<std::mutex> lk(S->ctx->mu);

@@ -1631,6 +1631,9 @@ constexpr int QSPLIT = 8;
 // its own, so that the atomics of the eight ranges do not queue on one line.
 constexpr int QSTRIDE = 64;
 constexpr int QCOUNTERS = QSPLIT * QSTRIDE;  // words of counters per launch
+// The range's first item and the one past its last, on the counter's next
+// line (read, never written, during the launch).
+constexpr int QLO = 32, QHI = 33;
 
 // Persistent launch: every wave repeatedly takes the next (image, tile)
 // item of a global queue until the queue is drained.  The launch's
@@ -1667,7 +1670,7 @@ struct MinWaves {
 template <int KIND, int NFP, bool REC, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MinWaves<KIND, NFP, REC, MODE>::value)))
 void k_persist(const DImg *__restrict__ imgs,
-                                                 const int2 *__restrict__ items, int n_items,
+                                                 const int2 *__restrict__ items,
                                                  unsigned int *__restrict__ counter,
                                                  const float4 *__restrict__ tf_all, int tf_bins, int wave_words)
 {
@@ -1696,8 +1699,8 @@ void k_persist(const DImg *__restrict__ imgs,
         unsigned int it = 0;
         if (lane == 0) it = atomicAdd(counter + part * QSTRIDE, 1u);
         it = (unsigned int)__builtin_amdgcn_readfirstlane((int)__shfl(it, 0));
-        const unsigned int lo = (unsigned int)(((int64_t)n_items * part) / QSPLIT);
-        const unsigned int hi = (unsigned int)(((int64_t)n_items * (part + 1)) / QSPLIT);
+        const unsigned int lo = (unsigned int)uni((int)counter[part * QSTRIDE + QLO]);
+        const unsigned int hi = (unsigned int)uni((int)counter[part * QSTRIDE + QHI]);
         if (it >= hi - lo) {
             if (--left == 0) break;
             part = (part + 1 == QSPLIT) ? 0 : part + 1;
