@@ -34,6 +34,7 @@
 #include "ytrc_host.h"
 #include "ytrc_kernels.h"
 #include "ytrc_pick.h"
+#include "ytrc_transfer.h"
 
 // Device memory of ytrc_render_noalloc: every staging buffer of one request
 // (its descriptor, brick order, extents, z-buffer, input image, output
@@ -438,6 +439,7 @@ struct Dataset {
     std::vector<DBrick> h_bricks;
     DBrick *d_bricks = nullptr;
     float *d_pool = nullptr;
+    size_t pool_cap = 0;  // bytes of its block
     uint8_t *d_masks = nullptr;
     uint64_t bytes = 0;
     int refs = 0;  // live batches and server requests that read it
@@ -446,6 +448,63 @@ struct Dataset {
 }  // namespace
 
 constexpr size_t PIN_BYTES = 2u << 20;
+constexpr size_t PIN_OUT = 4u << 20;
+constexpr int STOPS = 64, STOP_STRIDE = 16;
+
+// Device memory of dataset pools, batches and staged fields: freed blocks of
+// up to KEPT_BLOCK bytes are kept for the next one, KEPT_TOTAL in all.  A
+// program that renders frame after frame makes and frees the same blocks, and
+// an hipMalloc of 10 MB took up to 0.47 ms, an hipFree 0.07 ms, beside kernels
+// of 0.1 to 0.3 ms.  Used with ctx->mu held; a block is put back only when
+// nothing on the device uses it any more.
+struct DeviceBlocks {
+    static constexpr size_t KEPT_BLOCK = 32u << 20, KEPT_TOTAL = 96u << 20, KEPT_COUNT = 8;
+    std::vector<std::pair<char *, size_t>> kept;
+    size_t held = 0;
+
+    ~DeviceBlocks() { clear(); }
+    void clear()
+    {
+        for (auto &b : kept) hipFree(b.first);
+        kept.clear();
+        held = 0;
+    }
+    // A block of at least `bytes`: the smallest kept one that is no more than
+    // twice as large, else a new one.
+    hipError_t get(size_t bytes, char **p, size_t *cap)
+    {
+        int at = -1;
+        for (int i = 0; i < (int)kept.size(); i++) {
+            const size_t c = kept[(size_t)i].second;
+            if (c >= bytes && c / 2 <= bytes && (at < 0 || c < kept[(size_t)at].second)) at = i;
+        }
+        if (at >= 0) {
+            *p = kept[(size_t)at].first;
+            *cap = kept[(size_t)at].second;
+            held -= *cap;
+            kept.erase(kept.begin() + at);
+            return hipSuccess;
+        }
+        *p = nullptr;
+        *cap = bytes;
+        hipError_t e = hipMalloc((void **)p, bytes);
+        if (e == hipErrorOutOfMemory && !kept.empty()) {
+            (void)hipGetLastError();
+            clear();
+            e = hipMalloc((void **)p, bytes);
+        }
+        return e;
+    }
+    void put(char *p, size_t cap)
+    {
+        if (cap > KEPT_BLOCK || held + cap > KEPT_TOTAL || kept.size() >= KEPT_COUNT) {
+            hipFree(p);
+            return;
+        }
+        kept.push_back({p, cap});
+        held += cap;
+    }
+};
 
 struct ytrc_ctx {
     int device = 0;
@@ -458,9 +517,15 @@ struct ytrc_ctx {
     int n_cu = 0;
     size_t max_lds = 64 * 1024;  // LDS bytes one workgroup may allocate
     std::string name;            // marketing name and ISA of the device
-    char *pin = nullptr;         // PIN_BYTES of pinned host memory (staging of ytrc_render_noalloc)
+    char *pin = nullptr;         // pinned host memory of ytrc_render_noalloc: PIN_BYTES of staging, PIN_OUT of output
     char *scratch = nullptr;     // this device's `scratch` array (ytrc_render_noalloc)
     std::mutex *scratch_mu = nullptr;  // serialises the calls that share it
+    Transfer xfer;               // images to and fields from the caller's memory
+    DeviceBlocks blocks;
+    // Batches' stop flags, a line each in one page of pinned memory (an
+    // hipHostMalloc and its hipHostFree took 0.08 ms); those out of use.
+    int *stops = nullptr;
+    std::vector<int *> free_stops;
     std::map<int, Dataset> datasets;
     int next_ds = 1;
     std::mutex mu;
@@ -517,6 +582,7 @@ struct ytrc_batch {
     DImg *d_imgs = nullptr;
     char *arena = nullptr;
     uint64_t arena_bytes = 0;
+    size_t arena_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;  // persistent: the second stream's fork and join
     std::vector<hipEvent_t> ev_req;  // plain mode: before/after each request
@@ -532,6 +598,7 @@ struct ytrc_batch {
     double total_ms = 0.0;
     int timed = 0;
     std::vector<int> ds_ids;  // datasets this batch holds a reference on
+    bool own_stop = false;    // h_stop is an allocation of its own
     int *h_stop = nullptr;    // host-pinned stop flag read by the kernels (ytrc_batch_cancel)
     bool cancelled = false;   // the last launch was asked to stop: its images are incomplete
 };
@@ -645,6 +712,17 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 namespace {
 
+// Gives a batch's stop flag back (ctx->mu held).
+void release_stop(ytrc_batch *b)
+{
+    if (b->h_stop == nullptr) return;
+    if (b->own_stop)
+        hipHostFree(b->h_stop);
+    else
+        b->ctx->free_stops.push_back(b->h_stop);
+    b->h_stop = nullptr;
+}
+
 void dataset_release(ytrc_ctx *ctx, Dataset &ds);
 
 // Validates brick descriptors, lays out the point pool (stored_points per
@@ -708,8 +786,10 @@ int dataset_alloc(ytrc_ctx *ctx, const char *who, int n_bricks, const ytrc_brick
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, w + ": " + what + ": " + hipGetErrorString(e));
     };
-    hipError_t e = hipMalloc(&ds.d_pool, (size_t)pool_floats * 4);
+    char *pool = nullptr;
+    hipError_t e = ctx->blocks.get((size_t)pool_floats * 4, &pool, &ds.pool_cap);
     if (e != hipSuccess) return dev(e, "hipMalloc(pool)");
+    ds.d_pool = (float *)pool;
     if (mask_bytes > 0) {
         e = hipMalloc(&ds.d_masks, (size_t)mask_bytes);
         if (e != hipSuccess) return dev(e, "hipMalloc(masks)");
@@ -731,14 +811,29 @@ int dataset_alloc(ytrc_ctx *ctx, const char *who, int n_bricks, const ytrc_brick
 
 void dataset_release(ytrc_ctx *ctx, Dataset &ds)
 {
-    (void)ctx;
     if (ds.d_bricks) hipFree(ds.d_bricks);
-    if (ds.d_pool) hipFree(ds.d_pool);
+    if (ds.d_pool) ctx->blocks.put((char *)ds.d_pool, ds.pool_cap);
     if (ds.d_masks) hipFree(ds.d_masks);
     ds.d_bricks = nullptr;
     ds.d_pool = nullptr;
     ds.d_masks = nullptr;
 }
+
+// Device memory for fields on their way into a dataset, for as long as
+// ctx->mu is held; whoever used it has waited for the stream.
+struct Staging {
+    ytrc_ctx *ctx;
+    char *p = nullptr;
+    size_t cap = 0;
+
+    explicit Staging(ytrc_ctx *c) : ctx(c) {}
+    Staging(const Staging &) = delete;
+    ~Staging()
+    {
+        if (p) ctx->blocks.put(p, cap);
+    }
+    hipError_t get(size_t bytes) { return ctx->blocks.get(bytes, &p, &cap); }
+};
 
 int dataset_commit(ytrc_ctx *ctx, Dataset &ds, int32_t *ds_id_out)
 {
@@ -816,9 +911,17 @@ int ytrc_ctx_create(int32_t device, uint64_t budget_bytes, ytrc_ctx **out)
         return fail(YTRC_EDEVICE, std::string("ytrc_ctx_create: second stream: ") + hipGetErrorString(e));
     }
     int rc = scratch_setup(c);
-    if (rc == YTRC_OK && (e = hipHostMalloc((void **)&c->pin, PIN_BYTES, hipHostMallocDefault)) != hipSuccess)
+    if (rc == YTRC_OK && (e = hipHostMalloc((void **)&c->pin, PIN_BYTES + PIN_OUT, hipHostMallocDefault)) != hipSuccess)
         rc = fail(YTRC_EDEVICE, std::string("ytrc_ctx_create: pinned staging: ") + hipGetErrorString(e));
+    if (rc == YTRC_OK && (e = hipHostMalloc((void **)&c->stops, STOPS * STOP_STRIDE * sizeof(int),
+                                            hipHostMallocCoherent | hipHostMallocMapped)) != hipSuccess)
+        rc = fail(YTRC_EDEVICE, std::string("ytrc_ctx_create: stop flags: ") + hipGetErrorString(e));
+    for (int i = 0; rc == YTRC_OK && i < STOPS; i++) c->free_stops.push_back(c->stops + i * STOP_STRIDE);
+    if (rc == YTRC_OK && (e = c->xfer.open()) != hipSuccess)
+        rc = fail(YTRC_EDEVICE, std::string("ytrc_ctx_create: transfer buffers: ") + hipGetErrorString(e));
     if (rc != YTRC_OK) {
+        if (c->pin) hipHostFree(c->pin);
+        if (c->stops) hipHostFree(c->stops);
         hipStreamDestroy(c->stream2);
         hipStreamDestroy(c->stream);
         delete c;
@@ -834,12 +937,9 @@ void ytrc_ctx_destroy(ytrc_ctx *ctx)
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
     hipStreamSynchronize(ctx->stream2);
-    for (auto &kv : ctx->datasets) {
-        hipFree(kv.second.d_bricks);
-        hipFree(kv.second.d_pool);
-        if (kv.second.d_masks) hipFree(kv.second.d_masks);
-    }
+    for (auto &kv : ctx->datasets) dataset_release(ctx, kv.second);
     if (ctx->pin) hipHostFree(ctx->pin);
+    if (ctx->stops) hipHostFree(ctx->stops);
     hipStreamDestroy(ctx->stream2);
     hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -887,46 +987,74 @@ int ytrc_dataset_upload(ytrc_ctx *ctx, int32_t n_bricks, const ytrc_brick_desc *
     if (rc != YTRC_OK) return rc;
     // Each brick field goes to the device in C order as given (float64 or
     // float32) and k_store_field converts it to float32 in the device
-    // layout, fields interleaved per point.  One staging buffer holds the
-    // largest brick field; copies and kernels are ordered on the stream.
+    // layout, fields interleaved per point.  Fields are staged together, up
+    // to STAGE_MOST bytes or one field at a time; copies and kernels are
+    // ordered on the stream.
+    constexpr size_t STAGE_MOST = 32u << 20;
     const size_t esz = src_dtype == 0 ? 8 : 4;
-    int64_t max_np = 0;
+    auto points = [&](int b) {
+        const DBrick &h = ds.h_bricks[(size_t)b];
+        return (size_t)(h.dims[0] + h.vertex) * (size_t)(h.dims[1] + h.vertex) * (size_t)(h.dims[2] + h.vertex);
+    };
+    size_t most = 0, total = 0;
     for (int b = 0; b < n_bricks; b++) {
-        const DBrick &h = ds.h_bricks[b];
-        max_np = std::max(max_np, (int64_t)(h.dims[0] + h.vertex) * (h.dims[1] + h.vertex) *
-                                      (h.dims[2] + h.vertex));
+        most = std::max(most, points(b) * esz);
+        total += points(b) * esz * (size_t)n_fields;
     }
-    void *d_src = nullptr;
-    hipError_t e = hipMalloc(&d_src, (size_t)max_np * esz);
+    const size_t room = std::max(most, std::min(total, STAGE_MOST));
+    Staging stg(ctx);
+    hipError_t e = stg.get(room);
     if (e != hipSuccess) {
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, std::string("hipMalloc(staging): ") + hipGetErrorString(e));
     }
-    for (int b = 0; b < n_bricks && e == hipSuccess; b++) {
-        const DBrick &h = ds.h_bricks[b];
-        const int64_t np = (int64_t)(h.dims[0] + h.vertex) * (h.dims[1] + h.vertex) *
-                           (h.dims[2] + h.vertex);
+    struct Field {
+        int b, f;
+        size_t at;
+    };
+    std::vector<Field> group;
+    std::vector<Transfer::Piece> pieces;
+    size_t fill = 0;
+    auto store = [&](int b, int f, const char *src) {
+        const DBrick &h = ds.h_bricks[(size_t)b];
         const int64_t n = stored_points(h);
         const unsigned grid = (unsigned)((n + 255) / 256);
-        for (int f = 0; f < ds.nfp && e == hipSuccess; f++) {
-            const bool have = f < n_fields;
-            if (have)
-                e = hipMemcpyAsync(d_src, field_ptrs[(size_t)b * n_fields + f], (size_t)np * esz,
-                                   hipMemcpyHostToDevice, ctx->stream);
-            if (e != hipSuccess) break;
-            if (src_dtype == 0)
-                hipLaunchKernelGGL(k_store_field<double>, dim3(grid), dim3(256), 0, ctx->stream,
-                                   have ? (const double *)d_src : nullptr, ds.d_pool + h.data_off,
-                                   ds.nfp, f, h.dims[0], h.dims[1], h.dims[2], h.vertex, n);
-            else
-                hipLaunchKernelGGL(k_store_field<float>, dim3(grid), dim3(256), 0, ctx->stream,
-                                   have ? (const float *)d_src : nullptr, ds.d_pool + h.data_off,
-                                   ds.nfp, f, h.dims[0], h.dims[1], h.dims[2], h.vertex, n);
-            e = hipGetLastError();
+        if (src_dtype == 0)
+            hipLaunchKernelGGL(k_store_field<double>, dim3(grid), dim3(256), 0, ctx->stream, (const double *)src,
+                               ds.d_pool + h.data_off, ds.nfp, f, h.dims[0], h.dims[1], h.dims[2], h.vertex, n);
+        else
+            hipLaunchKernelGGL(k_store_field<float>, dim3(grid), dim3(256), 0, ctx->stream, (const float *)src,
+                               ds.d_pool + h.data_off, ds.nfp, f, h.dims[0], h.dims[1], h.dims[2], h.vertex, n);
+        return hipGetLastError();
+    };
+    auto flush = [&]() -> hipError_t {
+        hipError_t er;
+        {
+            std::lock_guard<std::mutex> lx(ctx->xfer.mu);
+            er = ctx->xfer.write(ctx->stream, pieces, stg.p);
         }
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(d_src);
+        for (const Field &g : group)
+            if (er == hipSuccess) er = store(g.b, g.f, stg.p + g.at);
+        group.clear();
+        pieces.clear();
+        fill = 0;
+        return er;
+    };
+    for (int b = 0; b < n_bricks && e == hipSuccess; b++)
+        for (int f = 0; f < ds.nfp && e == hipSuccess; f++) {
+            if (f >= n_fields) {
+                e = store(b, f, nullptr);
+                continue;
+            }
+            const size_t bytes = points(b) * esz;
+            if (fill + bytes > room) e = flush();
+            group.push_back({b, f, fill});
+            pieces.push_back({(const char *)field_ptrs[(size_t)b * n_fields + f], bytes});
+            fill += bytes;
+        }
+    if (e == hipSuccess) e = flush();
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = es;
     if (e != hipSuccess) {
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, std::string("ytrc_dataset_upload: ") + hipGetErrorString(e));
@@ -984,26 +1112,29 @@ int ytrc_dataset_build_vr(ytrc_ctx *ctx, int32_t n_grids, const ytrc_grid_desc *
     Dataset ds;
     int rc = dataset_alloc(ctx, who, n_leaves, bd.data(), n_fields, mask_ptrs, ds);
     if (rc != YTRC_OK) return rc;
-    void *d_cells = nullptr;
-    hipError_t e = hipMalloc(&d_cells, (size_t)cells * esz);
+    Staging stg(ctx);
+    hipError_t e = stg.get((size_t)cells * esz);
     if (e != hipSuccess) {
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, std::string("hipMalloc(cells): ") + hipGetErrorString(e));
     }
+    const char *const d_cells = stg.p;
     auto bail = [&](hipError_t err, const char *what) {
-        hipFree(d_cells);
+        hipStreamSynchronize(ctx->stream);
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, std::string(what) + ": " + hipGetErrorString(err));
     };
-    for (int g = 0; g < n_grids; g++) {
-        const size_t nc = (size_t)grids[g].dims[0] * grids[g].dims[1] * grids[g].dims[2];
-        for (int f = 0; f < n_fields; f++) {
-            e = hipMemcpyAsync((char *)d_cells + ((size_t)goff[(size_t)g] + (size_t)f * nc) * esz,
-                               cell_ptrs[(size_t)g * n_fields + f], nc * esz, hipMemcpyHostToDevice,
-                               ctx->stream);
-            if (e != hipSuccess) return bail(e, "hipMemcpyAsync(cells)");
+    {
+        std::vector<Transfer::Piece> pieces;
+        for (int g = 0; g < n_grids; g++) {
+            const size_t nc = (size_t)grids[g].dims[0] * grids[g].dims[1] * grids[g].dims[2];
+            for (int f = 0; f < n_fields; f++)
+                pieces.push_back({(const char *)cell_ptrs[(size_t)g * n_fields + f], nc * esz});
         }
+        std::lock_guard<std::mutex> lx(ctx->xfer.mu);
+        e = ctx->xfer.write(ctx->stream, pieces, stg.p);
     }
+    if (e != hipSuccess) return bail(e, "hipMemcpyAsync(cells)");
     int logmask = 0;
     for (int f = 0; f < n_fields; f++)
         if (log_fields != nullptr && log_fields[f]) logmask |= 1 << f;
@@ -1035,7 +1166,6 @@ int ytrc_dataset_build_vr(ytrc_ctx *ctx, int32_t n_grids, const ytrc_grid_desc *
     }
     e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return bail(e, "hipStreamSynchronize");
-    hipFree(d_cells);
     return dataset_commit(ctx, ds, ds_id_out);
 }
 
@@ -1075,10 +1205,8 @@ int ytrc_dataset_free(ytrc_ctx *ctx, int32_t ds_id)
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream2));
-    hipFree(it->second.d_bricks);
-    hipFree(it->second.d_pool);
-    if (it->second.d_masks) hipFree(it->second.d_masks);
     ctx->used -= it->second.bytes;
+    dataset_release(ctx, it->second);
     ctx->datasets.erase(it);
     return YTRC_OK;
 }
@@ -1560,28 +1688,58 @@ static inline double merge_input(int32_t kind, float o, double in)
     return o == (float)in ? in : (double)o;
 }
 
-// Copies a finished request's output (and image_in for channels it does
-// not write) into the caller's float64 (nv0, nv1, 4) image.
-int read_request_image(const ReqHost &q, const DImg &d, double *image_out)
+// The float64 pixels of a run of planes (each `stride` floats after the one
+// before it): o[4 p + c] from plane c, 0 for the channels past NCH.
+template <int NCH>
+void widen(const float *planes, int64_t stride, int n, double *o)
+{
+    for (int p = 0; p < n; p++)
+        for (int c = 0; c < 4; c++) o[4 * p + c] = c < NCH ? (double)planes[c * stride + p] : 0.0;
+}
+
+// Writes a run of a request's output (and image_in for channels it does not
+// write) into the caller's float64 (nv0, nv1, 4) image.
+struct ImageRun {
+    const double *in;
+    double *image_out;
+    int32_t kind;
+    int nch;
+
+    void operator()(int64_t first, int n, const float *planes, int64_t stride) const
+    {
+        double *o = image_out + 4 * first;
+        if (in != nullptr) {
+            const double *i4 = in + 4 * first;
+            for (int p = 0; p < n; p++)
+                for (int c = 0; c < 4; c++) {
+                    const double i = i4[4 * p + c];
+                    o[4 * p + c] = c < nch ? merge_input(kind, planes[c * stride + p], i) : i;
+                }
+        } else if (nch == 1) {
+            widen<1>(planes, stride, n, o);
+        } else if (nch == 2) {
+            widen<2>(planes, stride, n, o);
+        } else if (nch == 3) {
+            widen<3>(planes, stride, n, o);
+        } else {
+            widen<4>(planes, stride, n, o);
+        }
+    }
+};
+ImageRun image_run(const ReqHost &q, double *image_out)
+{
+    return {q.image_in.empty() ? nullptr : q.image_in.data(), image_out, q.r.kind, q.nch_out};
+}
+
+// Copies a finished request's image to the caller.
+int read_request_image(ytrc_ctx *ctx, const ReqHost &q, const DImg &d, double *image_out)
 {
     if (q.r.flags & YTRC_FLAG_PARTIAL)
         return fail(YTRC_EINVAL, "a YTRC_FLAG_PARTIAL request has a map, not an image: "
                                  "read it with ytrc_batch_read_partial");
-    std::vector<float> h((size_t)q.npix * q.nch_out);
-    HIPCHK(hipMemcpy(h.data(), d.out, sizeof(float) * h.size(), hipMemcpyDeviceToHost));
-    const bool has_in = !q.image_in.empty();
-    for (int64_t p = 0; p < q.npix; p++) {
-        for (int c = 0; c < 4; c++) {
-            const double in = has_in ? q.image_in[(size_t)p * 4 + c] : 0.0;
-            double v;
-            if (c < q.nch_out)
-                v = has_in ? merge_input(q.r.kind, h[(size_t)c * q.npix + p], in)
-                           : (double)h[(size_t)c * q.npix + p];
-            else
-                v = in;
-            image_out[(size_t)p * 4 + c] = v;
-        }
-    }
+    std::lock_guard<std::mutex> lk(ctx->xfer.mu);
+    HIPCHK(ctx->xfer.read(ctx->xfer.stream, d.out, q.npix, q.nch_out, image_out, 4 * sizeof(double),
+                          image_run(q, image_out)));
     return YTRC_OK;
 }
 
@@ -1618,10 +1776,10 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     for (int i = 0; i < n_req; i++) B->reqs[i] = P[i].q;
     auto bad = [&](int code, const std::string &m) {
         if (B->arena) {
-            hipFree(B->arena);
+            hipFree(B->arena);  // (it may hold copies under way)
             ctx->used -= B->arena_bytes;
         }
-        if (B->h_stop) hipHostFree(B->h_stop);
+        release_stop(B);
         if (B->ev0) hipEventDestroy(B->ev0);
         if (B->ev1) hipEventDestroy(B->ev1);
         if (B->ev_fork) hipEventDestroy(B->ev_fork);
@@ -1824,14 +1982,20 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     off = align_up(off + sizeof(DImg) * n_req, 256);
     if (ctx->budget != 0 && ctx->used + off > ctx->budget)
         return bad(YTRC_EBUDGET, "ytrc_batch_create: " + std::to_string(off) + " bytes exceed the HBM budget");
-    hipError_t e = hipMalloc(&B->arena, off);
+    hipError_t e = ctx->blocks.get(off, &B->arena, &B->arena_cap);
     if (e != hipSuccess) return bad(YTRC_EDEVICE, std::string("hipMalloc: ") + hipGetErrorString(e));
     B->arena_bytes = off;
     ctx->used += off;
     char *A = B->arena;
     // The stop flag: fine-grained pinned host memory that the kernels read
     // at system scope once per tile.
-    e = hipHostMalloc((void **)&B->h_stop, sizeof(int), hipHostMallocCoherent | hipHostMallocMapped);
+    if (!ctx->free_stops.empty()) {
+        B->h_stop = ctx->free_stops.back();
+        ctx->free_stops.pop_back();
+    } else {
+        e = hipHostMalloc((void **)&B->h_stop, sizeof(int), hipHostMallocCoherent | hipHostMallocMapped);
+        B->own_stop = true;
+    }
     if (e != hipSuccess) return bad(YTRC_EDEVICE, std::string("hipHostMalloc: ") + hipGetErrorString(e));
     __atomic_store_n(B->h_stop, 0, __ATOMIC_SEQ_CST);
     int *d_stop = nullptr;
@@ -2077,6 +2241,10 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
     DImg d;
     rc = stage_request(ctx, P, H, S, (const float4 *)(S + tf_off), 0, d);
     if (rc != YTRC_OK) return rc;
+    // The kernel's own stores take an image of up to PIN_OUT bytes straight
+    // to pinned memory, while it renders, instead of a copy after it.
+    const bool direct = sizeof(float) * (size_t)P.q.npix * P.q.nch_out <= PIN_OUT;
+    if (direct) d.out = (float *)(ctx->pin + PIN_BYTES);
     if (!P.tft.empty()) memcpy(Ht, P.tft.data(), sizeof(float4) * P.tft.size());
     // One request: the tiles in row order, cut into QSPLIT runs of equal
     // cost; with few of them, costly ones first within a run, as in a batch.
@@ -2132,7 +2300,10 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(s));
-    return read_request_image(P.q, d, image_out);
+    if (!direct) return read_request_image(ctx, P.q, d, image_out);
+    std::lock_guard<std::mutex> lx(ctx->xfer.mu);
+    ctx->xfer.read_here(d.out, P.q.npix, image_out, 4 * sizeof(double), image_run(P.q, image_out));
+    return YTRC_OK;
 }
 
 int ytrc_batch_request_ms(ytrc_batch *b, int32_t i, float *ms)
@@ -2216,7 +2387,7 @@ int ytrc_batch_read_image(ytrc_batch *b, int32_t i, double *image_out)
         return fail(YTRC_ECANCELLED, "ytrc_batch_read_image: the last launch was stopped; launch again");
     HIPCHK(hipSetDevice(b->ctx->device));
     HIPCHK(hipStreamSynchronize(b->ctx->stream));
-    return read_request_image(b->reqs[i], b->h_imgs[i], image_out);
+    return read_request_image(b->ctx, b->reqs[i], b->h_imgs[i], image_out);
 }
 
 int ytrc_batch_read_partial(ytrc_batch *b, int32_t i, double *map_out)
@@ -2297,10 +2468,11 @@ void ytrc_batch_destroy(ytrc_batch *b)
 {
     if (b == nullptr) return;
     hipSetDevice(b->ctx->device);
+    // (work on the second stream is joined to the first)
     hipStreamSynchronize(b->ctx->stream);
     if (b->arena) {
-        hipFree(b->arena);
         std::lock_guard<std::mutex> lk(b->ctx->mu);
+        b->ctx->blocks.put(b->arena, b->arena_cap);
         b->ctx->used -= b->arena_bytes;
     }
     {
@@ -2317,7 +2489,10 @@ void ytrc_batch_destroy(ytrc_batch *b)
     for (auto &e : b->ev_req) hipEventDestroy(e);
     if (b->gexec) hipGraphExecDestroy(b->gexec);
     if (b->graph) hipGraphDestroy(b->graph);
-    if (b->h_stop) hipHostFree(b->h_stop);
+    {
+        std::lock_guard<std::mutex> lk(b->ctx->mu);
+        release_stop(b);
+    }
     delete b;
 }
 
@@ -2941,7 +3116,7 @@ int ytrc_server_read(ytrc_server *S, int64_t id, double *image_out)
     if (it == S->reqs.end()) return fail(YTRC_EINVAL, "ytrc_server_read: unknown request");
     if (it->second.state != 2) return fail(YTRC_EINVAL, "ytrc_server_read: request is not finished");
     HIPCHK(hipSetDevice(S->ctx->device));
-    const int rc = read_request_image(it->second.P.q, it->second.d, image_out);
+    const int rc = read_request_image(S->ctx, it->second.P.q, it->second.d, image_out);
     srv_release(S, it->second);
     S->reqs.erase(it);
     return rc;
@@ -2958,14 +3133,20 @@ int ytrc_server_read_planar(ytrc_server *S, int64_t id, float *planes, int32_t c
     const ReqHost &q = it->second.P.q;
     if (cap_ch < q.nch_out) return fail(YTRC_EINVAL, "ytrc_server_read_planar: output has too few channels");
     HIPCHK(hipSetDevice(S->ctx->device));
-    HIPCHK(hipMemcpy(planes, it->second.d.out, sizeof(float) * (size_t)q.npix * q.nch_out,
-                     hipMemcpyDeviceToHost));
-    if (!q.image_in.empty())
-        for (int c = 0; c < q.nch_out; c++)
-            for (int64_t p = 0; p < q.npix; p++) {
-                float &o = planes[(size_t)c * q.npix + p];
-                o = (float)merge_input(q.r.kind, o, q.image_in[(size_t)p * 4 + c]);
-            }
+    const double *in = q.image_in.empty() ? nullptr : q.image_in.data();
+    {
+        std::lock_guard<std::mutex> lx(S->ctx->xfer.mu);
+        // (the planes lie back to back: one plane of all of them)
+        HIPCHK(S->ctx->xfer.read(S->ctx->xfer.stream, it->second.d.out, q.npix * q.nch_out, 1, planes, sizeof(float),
+                                 [&q, in, planes](int64_t first, int n, const float *from, int64_t) {
+                                     float *o = planes + first;
+                                     memcpy(o, from, sizeof(float) * (size_t)n);
+                                     if (in == nullptr) return;
+                                     for (int64_t i = first; i < first + n; i++)
+                                         planes[i] = (float)merge_input(q.r.kind, planes[i],
+                                                                        in[(size_t)(i % q.npix) * 4 + (size_t)(i / q.npix)]);
+                                 }));
+    }
     *nch = q.nch_out;
     srv_release(S, it->second);
     S->reqs.erase(it);
