@@ -1099,127 +1099,6 @@ struct IProjSampler {
     }
 };
 
-// IProjSampler for one field, under walk_vr_ctf_fast's conditions (walk_init
-// left every walking lane inside the brick, vertex blocks below 2^32 bytes,
-// strides of 24 bits).  The sub-samples of a visit lie symmetrically about
-// its mid-point, so the odd terms of the cubic along them cancel: with the
-// visit's length d and P = v_dir idds, their mean is
-//   V(mid) + d^2 (n^2 - 1) / (12 n^2) (fxy P0 P1 + fxz P0 P2 + fyz P1 P2),
-// fxy, fxz, fyz being the mixed partial derivatives at the mid-point: 27
-// FP32 operations instead of a cubic's coefficients and its power sums in
-// FP64.  The products with d and the sum stay in FP64.
-// 256^3 at 512^2: kernel 0.335 -> 0.292 ms, now 66 VALU and 23 SALU a visit
-// and about 9 lines looked up in L1 for each of its four loads; 2 or 6 visits
-// a round: 0.290 and 0.300.
-// The walk never depends on the data, so a round takes PF steps, issues
-// their loads together and then adds them in visit order (as
-// walk_projection_fast: steps past a ray's end read 0 at the out-of-range
-// offset, their lengths and positions stay finite).
-template <bool SHARED>
-__device__ __forceinline__ void walk_iproj_fast(Walk &w, double max_t, const BrickReg &b,
-                                                __amdgpu_buffer_rsrc_t rsrc, unsigned K0, unsigned K1,
-                                                const double (&pa)[3], const double (&pb)[3], float var,
-                                                double &sum)
-{
-    constexpr int PF = 4;
-    double t0 = w.tmax[0], t1 = w.tmax[1], t2 = w.tmax[2];
-    int c0 = w.cur[0], c1 = w.cur[1], c2 = w.cur[2];
-    double en = w.enter_t;
-    const int st0 = SHARED ? uni(w.step[0]) : w.step[0], st1 = SHARED ? uni(w.step[1]) : w.step[1],
-              st2 = SHARED ? uni(w.step[2]) : w.step[2];
-    const double td0 = SHARED ? uni_d(w.tdelta[0]) : w.tdelta[0], td1 = SHARED ? uni_d(w.tdelta[1]) : w.tdelta[1],
-                 td2 = SHARED ? uni_d(w.tdelta[2]) : w.tdelta[2];
-    const double sd0 = (st0 > 0) ? 1.0 : ((st0 < 0) ? -1.0 : 0.0);
-    const double sd1 = (st1 > 0) ? 1.0 : ((st1 < 0) ? -1.0 : 0.0);
-    const double sd2 = (st2 > 0) ? 1.0 : ((st2 < 0) ? -1.0 : 0.0);
-    K0 = (unsigned)uni((int)K0);
-    K1 = (unsigned)uni((int)K1);
-    double r0 = pb[0] - (double)c0, r1 = pb[1] - (double)c1, r2 = pb[2] - (double)c2;
-    const float P0 = (float)pa[0], P1 = (float)pa[1], P2 = (float)pa[2];
-    const float q01 = P0 * P1, q02 = P0 * P2, q12 = P1 * P2;
-    const float P01 = SHARED ? unif(q01) : q01, P02 = SHARED ? unif(q02) : q02, P12 = SHARED ? unif(q12) : q12;
-    const unsigned D0 = (unsigned)b.d0, D1 = (unsigned)b.d1, D2 = (unsigned)b.d2;
-    bool live = true;
-    double st = sum;
-    while (live) {
-        unsigned off[PF];
-        float x[PF], y[PF], z[PF];
-        double d[PF];
-#pragma unroll
-        for (int u = 0; u < PF; u++) {
-            const bool a01 = t0 < t1;
-            const double m = min_f64(t0, t1);
-            const bool bm = m < t2;
-            const double tm = min_f64(m, t2);
-            const bool ge = tm >= max_t;
-            const double ex = min_f64(tm, max_t);
-            const unsigned o = __umul24((unsigned)c0 >> 2, K0) +
-                               (__umul24((unsigned)c1 >> 2, K1) +
-                                (__umul24((unsigned)c2 >> 2, VK2) +
-                                 (__umul24((unsigned)c0, VW0) + (__umul24((unsigned)c1, VW1) + ((unsigned)c2 << 2)))));
-            off[u] = live ? o : 0xffffff00u;
-            d[u] = ex - en;
-            const double mid = __builtin_fma(0.5, d[u], en);
-            x[u] = (float)__builtin_fma(mid, pa[0], r0);
-            y[u] = (float)__builtin_fma(mid, pa[1], r1);
-            z[u] = (float)__builtin_fma(mid, pa[2], r2);
-            // formed at their step: none of its FP64 times stay live
-            asm volatile("" : "+v"(off[u]), "+v"(x[u]), "+v"(y[u]), "+v"(z[u]), "+v"(d[u]));
-            bool out;
-            if (bm) {
-                if (a01) {
-                    asm volatile("");
-                    c0 += st0;
-                    t0 += td0;
-                    r0 -= sd0;
-                    out = (unsigned)c0 >= D0;
-                } else {
-                    asm volatile("");
-                    c1 += st1;
-                    t1 += td1;
-                    r1 -= sd1;
-                    out = (unsigned)c1 >= D1;
-                }
-            } else {
-                asm volatile("");
-                c2 += st2;
-                t2 += td2;
-                r2 -= sd2;
-                out = (unsigned)c2 >= D2;
-            }
-            en = tm;
-            live = live & !(out | ge);
-        }
-        float cv[PF][8];
-#pragma unroll
-        for (int u = 0; u < PF; u++) {
-            BufLoad<2>::get(rsrc, off[u], cv[u]);
-            BufLoad<2>::get(rsrc, off[u] + 4u * vcorner(0, 1, 0), cv[u] + 2);
-            BufLoad<2>::get(rsrc, off[u] + 4u * vcorner(1, 0, 0), cv[u] + 4);
-            BufLoad<2>::get(rsrc, off[u] + 4u * vcorner(1, 1, 0), cv[u] + 6);
-        }
-#pragma unroll
-        for (int u = 0; u < PF; u++) {
-            const float *c = cv[u];
-            // along z, then y, then x
-            const float z00 = c[1] - c[0], z01 = c[3] - c[2], z10 = c[5] - c[4], z11 = c[7] - c[6];
-            const float e00 = __builtin_fmaf(z00, z[u], c[0]), e01 = __builtin_fmaf(z01, z[u], c[2]);
-            const float e10 = __builtin_fmaf(z10, z[u], c[4]), e11 = __builtin_fmaf(z11, z[u], c[6]);
-            const float g0 = e01 - e00, g1 = e11 - e10;
-            const float h0 = __builtin_fmaf(g0, y[u], e00), h1 = __builtin_fmaf(g1, y[u], e10);
-            const float v = __builtin_fmaf(h1 - h0, x[u], h0);
-            const float m0 = z01 - z00, D = (z11 - z10) - m0;
-            const float fxy = g1 - g0;
-            const float fyz = __builtin_fmaf(D, x[u], m0), fxz = __builtin_fmaf(D, y[u], z10 - z00);
-            const float df = (float)d[u];
-            const float mean = __builtin_fmaf(
-                df * df * var, __builtin_fmaf(fxy, P01, __builtin_fmaf(fxz, P02, fyz * P12)), v);
-            st = __builtin_fma((double)mean, d[u], st);
-        }
-    }
-    sum = st;
-}
-
 // walk_loop for a sampler of one vertex-centred field (S::sample; volume
 // renders with grey opacity), under
 // walk_vr_ctf_fast's conditions (walk_init left every walking lane inside
@@ -1604,16 +1483,7 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
 #pragma unroll
                 for (int c = 0; c < 3; c++) s.st[c] = st[c];
                 s.rec = &rec;
-                bool fastw = false;
-                if constexpr (!REC && NFP == 1) {
-                    const VertexFast vf = vertex_fast(s.b, w);
-                    if (vf.ok) {
-                        walk_iproj_fast<!PP>(w, max_t, s.b, brick_rsrc(s.data, vf.bytes), vf.k0, vf.k1, s.pa, s.pb,
-                                             unif((float)((ns * ns - 1.0) / (12.0 * ns * ns))), s.st[0]);
-                        fastw = true;
-                    }
-                }
-                if (!fastw) walk_loop(b, w, max_t, s);
+                walk_loop(b, w, max_t, s);
 #pragma unroll
                 for (int c = 0; c < 3; c++) st[c] = s.st[c];
             } else {
@@ -1781,7 +1651,6 @@ constexpr int QLO = 32, QHI = 33;
 //   faster than 4, and 7 waves (72 VGPRs, 68-byte spill) 0.5 % slower;
 // - the same with grey opacity: 4 (128 VGPRs); 5 and 6 waves were 0 to 9 %
 //   slower;
-// - interpolated projection, one field: 4 (111 VGPRs with 4 visits a round);
 // - projection, one field, no record: 3.6 % faster than the 5 waves its
 //   90 VGPRs give;
 // - projection, two fields (item x weight and weight): 4 (128 VGPRs) instead
@@ -1795,7 +1664,6 @@ struct MinWaves {
                                  : (KIND == 1 && (MODE == 1 || MODE == 3 || MODE == 19)) ? 6
                                  : (KIND == 1 && (MODE & 32) != 0)                       ? 4
                                  : (KIND == 0)                                           ? 6
-                                 : (KIND == 2)                                           ? 4
                                                                                          : 1;
 };
 
