@@ -364,6 +364,39 @@ bool few_items(int n_cu, int kind, int64_t n)
     return n < (kind == YTRC_PROJECTION ? slots : 4 * slots);
 }
 
+// How many of an image's longest chains of visits all its tiles' chains make
+// (from tile_costs, without its constant part).
+double chains(const std::vector<float> &cost)
+{
+    double sum = 0.0, most = 0.0;
+    for (float c : cost) {
+        sum += c;
+        most = std::max(most, (double)c);
+    }
+    const double base = most / 33.0;
+    return most > 0.0 ? (sum - base * (double)cost.size()) / (most - base) : 0.0;
+}
+
+// The kernel that takes four waves to a tile (k_split) for a request in a
+// launch of `chains` chains in all, nullptr where one wave a tile is as fast.
+// Four waves shorten the longest chains, which is what counts while the
+// chains fill the chip's SIMDs about once; beyond that the steps they repeat
+// cost more.  Time of one wave over time of four, by chains per SIMD (volume
+// renders of 48^3 to 256^3, widths 0.7 to 1.9, 200^2 to 1024^2):
+//   one brick       0.1 to 0.6: 1.3 to 2.0, 0.9: 1.15 to 1.34, 1.3: 1.08 to
+//                   1.11, 1.8: 0.87 to 1.26, 2.1: 0.87
+//   per-pixel lens  0.2: 1.5 to 2.1, 0.8: 1.2 to 1.34, 1.3: 1.02 to 1.2, 2.0: 0.84
+//   more bricks     (whose rays' ends fill rounds badly) 0.2: 1.4 to 1.8, 0.5:
+//                   1.41, 0.6: 1.38, 0.9: 1.07 to 1.11, 1.2: 0.89
+pfn_t split_kernel(int n_cu, int kind, int nfp, bool rec, int mode, int n_order, double chains)
+{
+    if (nfp != 1 || rec) return nullptr;
+    const double most = n_order == 1 ? 1.25 : 0.75;
+    return chains <= most * 4.0 * n_cu ? pick_split(kind, mode) : nullptr;
+}
+// LDS of k_split after its tables: two rounds' opacities, and the item.
+constexpr size_t SPLIT_LDS = sizeof(float) * SPLIT_Q + 16;
+
 // Words of LDS per wave that a persistent launch gives after its tables
 // (k_persist's wave_words): the vertex-block buffer with mode bit 4, a
 // projection's table of offset terms (walk_projection_fast).
@@ -565,6 +598,7 @@ struct PGroup {
     int nfp = 1;
     bool rec = false;
     pfn_t fn = nullptr;
+    pfn_t split = nullptr;  // its k_split, where the batch has few tiles
     int n_items = 0;
     const int2 *items = nullptr;
     int counter = 0;
@@ -1890,6 +1924,12 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     std::vector<std::vector<int2>> gitems;
     std::vector<std::array<int, QSPLIT + 1>> gbounds;
     std::vector<size_t> gitems_off;
+    std::vector<std::vector<float>> costs((size_t)n_req);
+    double chains_all = 0.0;  // the launches run side by side
+    for (int i = 0; i < n_req; i++) {
+        costs[(size_t)i] = tile_costs(reqs[i], ctx->datasets[reqs[i].ds_id].h_bricks.data(), P[i].tsh);
+        chains_all += chains(costs[(size_t)i]);
+    }
     for (size_t L = 0; L < plans.size(); L++) {
         std::vector<int> ids = plans[L].ids;
         std::stable_sort(ids.begin(), ids.end(),
@@ -1911,16 +1951,17 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         for (int i : ids) ntiles += P[i].q.ntiles;
         const bool costly_first = z && few_items(ctx->n_cu, std::get<0>(plans[L].variant), ntiles);
         std::vector<std::vector<int>> zord(ids.size());
-        std::vector<std::vector<float>> cost(ids.size());
+        std::vector<const float *> cost(ids.size());
         std::vector<float> most(ids.size());
         std::vector<std::array<int, QSPLIT + 1>> cut(ids.size());
         for (size_t o = 0; o < ids.size(); o++) {
             const PrepReq &Q = P[ids[o]];
             const int th = 64 >> Q.tsh, tw = 1 << Q.tsh;
             if (z) zord[o] = tiles_z_order((Q.q.r.nv[0] + th - 1) / th, (Q.q.r.nv[1] + tw - 1) / tw);
-            cost[o] = tile_costs(reqs[ids[o]], ctx->datasets[reqs[ids[o]].ds_id].h_bricks.data(), Q.tsh);
-            most[o] = *std::max_element(cost[o].begin(), cost[o].end());
-            equal_cost_runs(cost[o], zord[o], cut[o].data());
+            const std::vector<float> &c = costs[(size_t)ids[o]];
+            cost[o] = c.data();
+            most[o] = *std::max_element(c.begin(), c.end());
+            equal_cost_runs(c, zord[o], cut[o].data());
         }
         for (int r = 0; r < QSPLIT; r++) {
             bounds[(size_t)r] = (int)items.size();
@@ -1953,6 +1994,10 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         g.rec = std::get<2>(plans[L].variant) != 0;
         g.mode = std::get<3>(plans[L].variant);
         g.fn = pick_persist(g.kind, g.nfp, g.rec, g.mode);
+        g.split = g.fn;
+        for (int i : ids)
+            if (g.split != nullptr)
+                g.split = split_kernel(ctx->n_cu, g.kind, g.nfp, g.rec, g.mode, P[i].q.r.n_order, chains_all);
         g.n_items = (int)items.size();
         g.counter = (int)B->groups.size();
         g.tf_base = plan_base[L];
@@ -1960,6 +2005,13 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         g.lds = has_tf(g.kind) ? sizeof(float4) * (size_t)g.tf_bins : 0;
         // up to 4 waves' buffers follow the tables
         const size_t lds_most = g.lds + 4 * sizeof(unsigned) * required_wave_words(g.kind, g.nfp, g.rec, g.mode);
+        if (g.lds + SPLIT_LDS > ctx->max_lds) g.split = nullptr;
+        if (g.split != nullptr && g.lds + SPLIT_LDS > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute((const void *)g.split, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)(g.lds + SPLIT_LDS));
+            if (e != hipSuccess)
+                return bad(YTRC_EDEVICE, std::string("ytrc_batch_create: hipFuncSetAttribute: ") + hipGetErrorString(e));
+        }
         if (lds_most > ctx->max_lds)
             return bad(YTRC_EINVAL, "ytrc_batch_create: the distinct transfer functions of one launch need " +
                                         std::to_string(lds_most) + " B of LDS, more than the " +
@@ -2121,17 +2173,20 @@ int enqueue_persistent(ytrc_batch *b, hipStream_t s)
         PGroup &g = b->groups[order[k]];
         hipStream_t gs = (k == 0) ? s : b->ctx->stream2;
         // each wave's buffer after the tables
-        const int ww = required_wave_words(g.kind, g.nfp, g.rec, g.mode);
-        const size_t lds = g.lds + (size_t)b->waves_per_group * ww * sizeof(unsigned);
+        const bool split = g.split != nullptr && b->waves_per_group == NSEG;
+        const pfn_t fn = split ? g.split : g.fn;
+        const int ww = split ? 0 : required_wave_words(g.kind, g.nfp, g.rec, g.mode);
+        const size_t lds = g.lds + (split ? SPLIT_LDS : (size_t)b->waves_per_group * ww * sizeof(unsigned));
+        const int per_group = split ? 1 : b->waves_per_group;  // items at a time
         int per_cu = b->groups_per_cu;
         if (per_cu == 0) {
             int nb = 0;
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, g.fn, threads, lds));
+            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, threads, lds));
             per_cu = std::max(1, (fork && k == 0) ? nb - 1 : nb);
         }
         g.grid = std::max(1, std::min(per_cu * b->ctx->n_cu,
-                                      (g.n_items + b->waves_per_group - 1) / b->waves_per_group));
-        hipLaunchKernelGGL(g.fn, dim3(g.grid), dim3(threads), lds, gs, (const DImg *)b->d_imgs,
+                                      (g.n_items + per_group - 1) / per_group));
+        hipLaunchKernelGGL(fn, dim3(g.grid), dim3(threads), lds, gs, (const DImg *)b->d_imgs,
                            g.items, b->counters + (size_t)g.counter * QCOUNTERS, b->tf_all + g.tf_base,
                            g.tf_bins, ww);
         HIPCHK(hipGetLastError());
@@ -2250,9 +2305,11 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
     // cost; with few of them, costly ones first within a run, as in a batch.
     int2 *items = (int2 *)(Ht + (items_off - tf_off));
     int cut[QSPLIT + 1];
+    double nchains = 0.0;
     {
         const std::vector<float> cost = tile_costs(*req, ctx->datasets[req->ds_id].h_bricks.data(), P.tsh);
         equal_cost_runs(cost, {}, cut);
+        nchains = chains(cost);
         if (few_items(ctx->n_cu, req->kind, P.q.ntiles)) {
             const float most = *std::max_element(cost.begin(), cost.end());
             for (int r = 0; r < QSPLIT; r++) {
@@ -2270,11 +2327,17 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
     memset(queue, 0, sizeof(unsigned int) * QCOUNTERS);
     set_bounds(queue, cut);
     memcpy(Ht + (img_off - tf_off), &d, sizeof(DImg));
-    const pfn_t fn = pick_persist(req->kind, P.q.nfp, false, P.q.mode);
+    pfn_t fn = pick_persist(req->kind, P.q.nfp, false, P.q.mode);
     if (fn == nullptr) return fail(YTRC_ENOTIMPL, "ytrc_render_noalloc: no kernel for this request");
     const int wpg = 4, threads = 64 * wpg;
-    const int ww = required_wave_words(req->kind, P.q.nfp, false, P.q.mode);
-    const size_t lds = (has_tf(req->kind) ? sizeof(float4) * P.tft.size() : 0) + (size_t)wpg * ww * sizeof(unsigned);
+    const size_t tables = has_tf(req->kind) ? sizeof(float4) * P.tft.size() : 0;
+    const pfn_t sfn = tables + SPLIT_LDS <= ctx->max_lds
+                          ? split_kernel(ctx->n_cu, req->kind, P.q.nfp, false, P.q.mode, req->n_order, nchains)
+                          : nullptr;
+    const bool split = sfn != nullptr;
+    if (split) fn = sfn;
+    const int ww = split ? 0 : required_wave_words(req->kind, P.q.nfp, false, P.q.mode);
+    const size_t lds = tables + (split ? SPLIT_LDS : (size_t)wpg * ww * sizeof(unsigned));
     if (lds > 64 * 1024)
         HIPCHK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipStream_t s = ctx->stream;
@@ -2293,7 +2356,8 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
     if (P.q.ntiles > 0) {
         int nb = 0;
         HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, threads, lds));
-        const int grid = std::max(1, std::min(std::max(1, nb) * ctx->n_cu, (P.q.ntiles + wpg - 1) / wpg));
+        const int per_group = split ? 1 : wpg;  // tiles at a time
+        const int grid = std::max(1, std::min(std::max(1, nb) * ctx->n_cu, (P.q.ntiles + per_group - 1) / per_group));
         hipLaunchKernelGGL(fn, dim3(grid), dim3(threads), lds, s, (const DImg *)(S + img_off),
                            (const int2 *)(S + items_off), counters,
                            (const float4 *)(S + tf_off), (int)P.tft.size(), ww);

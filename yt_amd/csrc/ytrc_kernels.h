@@ -613,10 +613,9 @@ __device__ __forceinline__ bool quad_visit_ok(const float (&k)[4])
 // relative precision; the FP64 transmittance st then takes T (1 - Q) once
 // per visit.
 template <int NS>
-__device__ __forceinline__ void ctf_visit(const TFCache &tf, const float4 *__restrict__ lt,
-                                          const float (&ku)[4], float dtf, int ns, double (&st)[4])
+__device__ __forceinline__ void ctf_opacity(const TFCache &tf, const float4 *__restrict__ lt,
+                                            const float (&ku)[4], float dtf, int ns, float (&Q)[3])
 {
-    float Q[3] = {0.0f, 0.0f, 0.0f};
     float G[3] = {dtf, dtf, dtf};
     const int nsq = (NS > 0) ? NS : ns;
     float sf = 0.0f;
@@ -635,6 +634,13 @@ __device__ __forceinline__ void ctf_visit(const TFCache &tf, const float4 *__res
             G[ch] = __builtin_fmaf(-dtf, Q[ch], dtf);
         }
     }
+}
+template <int NS>
+__device__ __forceinline__ void ctf_visit(const TFCache &tf, const float4 *__restrict__ lt,
+                                          const float (&ku)[4], float dtf, int ns, double (&st)[4])
+{
+    float Q[3] = {0.0f, 0.0f, 0.0f};
+    ctf_opacity<NS>(tf, lt, ku, dtf, ns, Q);
 #pragma unroll
     for (int ch = 0; ch < 3; ch++) st[ch] = __builtin_fma(-st[ch], (double)Q[ch], st[ch]);
 }
@@ -1195,6 +1201,184 @@ __device__ __forceinline__ VertexFast vertex_fast(const BrickReg &b, const Walk 
             (unsigned)k0, (unsigned)k1};
 }
 
+// Waves that share a tile in k_split, visits of a round that each of them
+// samples, and the visits of a round.
+constexpr int NSEG = 4, SPLIT_B = 4, SPLIT_R = NSEG * SPLIT_B;
+// LDS floats of k_split after its tables: two rounds' opacities.
+constexpr int SPLIT_Q = 2 * SPLIT_R * 3 * 64;
+
+// A brick's walk by the NSEG waves of a workgroup, all on the same rays: in
+// each round of SPLIT_R visits wave `seg` samples SPLIT_B and steps over the
+// others, the visits' opacities meet in LDS (qbuf, two rounds in turn, `par`
+// the present one), and waves 0, 1 and 2 take one channel's transmittance T
+// through them in the order of the visits: the FP64 products are those of
+// one wave's walk, in its order, so the same image bit for bit.  A lane past
+// its end leaves opacity 0, which changes no T.  Every wave of the workgroup
+// calls it with the same rays, whose steps do not depend on what it samples,
+// so all of them take the same rounds and meet the same barriers.
+// SHARED: one direction, walk_vr_ctf_fast's arithmetic; else VRSampler's.
+template <int NS, bool SHARED, class S>
+__device__ __forceinline__ void walk_vr_ctf_split(Walk &w, bool live, double max_t, const S &smp,
+                                                  __amdgpu_buffer_rsrc_t rsrc, unsigned K0, unsigned K1,
+                                                  const uint8_t *mask, const TFCache &tf,
+                                                  const float4 *__restrict__ lt, int seg, int lane, float *qbuf,
+                                                  int &par, double &T)
+{
+    const BrickReg &b = smp.b;
+    double t0 = w.tmax[0], t1 = w.tmax[1], t2 = w.tmax[2];
+    int c0 = w.cur[0], c1 = w.cur[1], c2 = w.cur[2];
+    double en = w.enter_t;
+    // (where the direction is shared, from a lane that walks: walk_init leaves
+    // the others' increments unset)
+    const int from = __builtin_ctzll(__ballot(live));
+    auto lane_i = [&](int x) { return SHARED ? __builtin_amdgcn_readlane(x, from) : x; };
+    auto lane_d = [&](double x) {
+        if (!SHARED) return x;
+        const uint64_t u = (uint64_t)__double_as_longlong(x);
+        const uint64_t lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, from);
+        const uint64_t hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), from);
+        return __longlong_as_double((long long)((hi << 32) | lo));
+    };
+    const int st0 = lane_i(w.step[0]), st1 = lane_i(w.step[1]), st2 = lane_i(w.step[2]);
+    const double td0 = lane_d(w.tdelta[0]), td1 = lane_d(w.tdelta[1]), td2 = lane_d(w.tdelta[2]);
+    K0 = (unsigned)uni((int)K0);
+    K1 = (unsigned)uni((int)K1);
+    // (walk_vr_ctf_fast's cell-relative positions, stepped as there: their
+    // rounding is part of the image)
+    const double sd0 = (st0 > 0) ? 1.0 : ((st0 < 0) ? -1.0 : 0.0);
+    const double sd1 = (st1 > 0) ? 1.0 : ((st1 < 0) ? -1.0 : 0.0);
+    const double sd2 = (st2 > 0) ? 1.0 : ((st2 < 0) ? -1.0 : 0.0);
+    double r0 = smp.pb[0] - (double)c0, r1 = smp.pb[1] - (double)c1, r2 = smp.pb[2] - (double)c2;
+    const double hns = 0.5 * smp.inv_ns;
+    const float inv_nsf = unif((float)smp.inv_ns);
+    const float P0 = smp.paf[0], P1 = smp.paf[1], P2 = smp.paf[2];
+    const float P01 = P0 * P1, P02 = P0 * P2, P12 = P1 * P2;
+    const float P012 = P01 * P2;
+    const float idb = tf.idbin, qc1 = tf.qc1;
+    const unsigned D0 = (unsigned)b.d0, D1 = (unsigned)b.d1, D2 = (unsigned)b.d2;
+    const int ns = smp.n_samples;
+    int v = 0;  // of the round
+    while (__any(live)) {
+        // one visit: sampled by this wave or stepped over
+        const bool mine = (v >> 2) == seg;  // (uniform; SPLIT_B is 4)
+        const bool a01 = t0 < t1;
+        const double m = min_f64(t0, t1);
+        const bool bm = m < t2;
+        const double tm = min_f64(m, t2);
+        const bool ge = tm >= max_t;
+        if (mine) {
+            float Q[3] = {0.0f, 0.0f, 0.0f};
+            if (live) {
+                const double ex = min_f64(tm, max_t);
+                const unsigned o = __umul24((unsigned)c0 >> 2, K0) +
+                                   (__umul24((unsigned)c1 >> 2, K1) +
+                                    (__umul24((unsigned)c2 >> 2, VK2) +
+                                     (__umul24((unsigned)c0, VW0) + (__umul24((unsigned)c1, VW1) + ((unsigned)c2 << 2)))));
+                int mval = 1;
+                if (mask != nullptr) mval = mask[(int)__umul24(__umul24(c0, D1) + c1, D2) + c2];
+                float cv[8];
+                BufLoad<2>::get(rsrc, o, cv);
+                BufLoad<2>::get(rsrc, o + 4u * vcorner(0, 1, 0), cv + 2);
+                BufLoad<2>::get(rsrc, o + 4u * vcorner(1, 0, 0), cv + 4);
+                BufLoad<2>::get(rsrc, o + 4u * vcorner(1, 1, 0), cv + 6);
+                const double d = ex - en;
+                float ku[4], k0, dtf;
+                if constexpr (SHARED) {
+                    const double tt = __builtin_fma(d, hns, en);
+                    const float x0 = (float)__builtin_fma(tt, smp.pa[0], r0);
+                    const float y0 = (float)__builtin_fma(tt, smp.pa[1], r1);
+                    const float z0 = (float)__builtin_fma(tt, smp.pa[2], r2);
+                    dtf = (float)d * inv_nsf;
+                    const float A = cv[0];
+                    const float Bz = cv[1] - cv[0], e1 = cv[3] - cv[2], e2 = cv[5] - cv[4], e3 = cv[7] - cv[6];
+                    const float By = cv[2] - cv[0], g1 = cv[6] - cv[4];
+                    const float Cyz = e1 - Bz, g3 = e3 - e2;
+                    const float Bx = cv[4] - cv[0], Cxy = g1 - By, Cxz = e2 - Bz, D = g3 - Cyz;
+                    const float fxy = __builtin_fmaf(D, z0, Cxy);
+                    const float fxz = __builtin_fmaf(D, y0, Cxz);
+                    const float fyz = __builtin_fmaf(D, x0, Cyz);
+                    const float tyz = __builtin_fmaf(Cyz, z0, By);
+                    const float fx = __builtin_fmaf(y0, fxy, __builtin_fmaf(Cxz, z0, Bx));
+                    const float fy = __builtin_fmaf(x0, fxy, tyz);
+                    const float fz = __builtin_fmaf(x0, fxz, __builtin_fmaf(Cyz, y0, Bz));
+                    k0 = __builtin_fmaf(x0, fx, __builtin_fmaf(y0, tyz, __builtin_fmaf(z0, Bz, A)));
+                    const float q1 = dtf * idb, q2 = q1 * dtf, q3 = q2 * dtf;
+                    ku[0] = __builtin_fmaf(k0, idb, qc1);
+                    ku[1] = __builtin_fmaf(fx, P0, __builtin_fmaf(fy, P1, fz * P2)) * q1;
+                    ku[2] = __builtin_fmaf(fxy, P01, __builtin_fmaf(fxz, P02, fyz * P12)) * q2;
+                    ku[3] = D * P012 * q3;
+                } else {
+                    // VRSampler::sample
+                    const double dt = d * smp.inv_ns;
+                    const double tt = en + 0.5 * dt;
+                    const float dtf0 = (float)dt;
+                    float dp[3], ds[3], k[4];
+#pragma unroll
+                    for (int i = 0; i < 3; i++) {
+                        const double ci = (double)(i == 0 ? c0 : (i == 1 ? c1 : c2));
+                        dp[i] = (float)(__builtin_fma(tt, smp.pa[i], smp.pb[i]) - ci);
+                        ds[i] = smp.paf[i] * dtf0;
+                    }
+                    trilinear_cubic(cv, dp, ds, k);
+                    dtf = dtf0;
+                    k0 = k[0];
+                    ku[0] = __builtin_fmaf(k[0], idb, qc1);
+                    ku[1] = k[1] * idb, ku[2] = k[2] * idb, ku[3] = k[3] * idb;
+                    // (quad_visit_ok takes the coefficients as they are)
+                    if (!quad_visit_ok(k)) mval = 0;
+                }
+                bool fine = mval == 1;
+                if constexpr (SHARED) {
+                    const float mm = __builtin_fabsf(k0) + __builtin_fabsf(ku[1]) + __builtin_fabsf(ku[2]) +
+                                     __builtin_fabsf(ku[3]);
+                    fine = fine && __builtin_amdgcn_classf(mm, (1 << 7) | (1 << 8));
+                }
+                if (fine) ctf_opacity<NS>(tf, lt, ku, dtf, ns, Q);
+            }
+            float *q = qbuf + (par * SPLIT_R + v) * 192 + lane;
+            q[0] = Q[0];
+            q[64] = Q[1];
+            q[128] = Q[2];
+        }
+        if (live) {
+            bool out;
+            if (bm) {
+                if (a01) {
+                    asm volatile("");
+                    c0 += st0;
+                    t0 += td0;
+                    if constexpr (SHARED) r0 -= sd0;
+                    out = (unsigned)c0 >= D0;
+                } else {
+                    asm volatile("");
+                    c1 += st1;
+                    t1 += td1;
+                    if constexpr (SHARED) r1 -= sd1;
+                    out = (unsigned)c1 >= D1;
+                }
+            } else {
+                asm volatile("");
+                c2 += st2;
+                t2 += td2;
+                if constexpr (SHARED) r2 -= sd2;
+                out = (unsigned)c2 >= D2;
+            }
+            en = tm;
+            live = !(out || ge);
+        }
+        if (++v == SPLIT_R || !__any(live)) {
+            // the round is over: v visits, the same in every wave
+            __syncthreads();
+            if (seg < 3) {
+                const float *q = qbuf + par * SPLIT_R * 192 + seg * 64 + lane;
+                for (int i = 0; i < v; i++) T = __builtin_fma(-T, (double)q[i * 192], T);
+            }
+            par ^= 1;
+            v = 0;
+        }
+    }
+}
+
 // LightSourceRenderSampler.sample (image_samplers.pyx:548-590) with
 // FIT_eval_transfer_with_light (field_interpolation_tables.pxd:115-143): per
 // sub-sample the tables' values, the gradient of field 0 normalised and
@@ -1295,9 +1479,12 @@ struct LightSampler {
 
 // Casts the rays of one 8x8 tile of image `im` through its bricks.  `im`
 // and `tile` are wave-uniform.
-template <int KIND, int NFP, bool REC, int MODE>
+// SPLIT (k_split): the NSEG waves of the workgroup call it together for one
+// tile; wave seg < 3 holds and writes channel seg.
+template <int KIND, int NFP, bool REC, int MODE, bool SPLIT = false>
 __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
-                                            const float4 *lt, float *wbuf = nullptr, int wave_words = 0)
+                                            const float4 *lt, float *wbuf = nullptr, int wave_words = 0,
+                                            int seg = 0, int *par = nullptr)
 {
     const int tsh = im.tsh;
     const int tw = 1 << tsh, th = 64 >> tsh;
@@ -1368,6 +1555,7 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
 #pragma unroll
         for (int c = 0; c < 3; c++) st[c] = 1.0 - st[c];
     }
+    if constexpr (SPLIT) st[0] = seg == 0 ? st[0] : (seg == 1 ? st[1] : st[2]);
 
     // Early ray termination (YTRC_FLAG_ERT, VR only): the reference composites
     // each new sample on top as t grows (field_interpolation_tables.pxd:107-110),
@@ -1401,6 +1589,39 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
         const DBrick &b = im.bricks[bid];
         Walk w;
         if (go) go = walk_init<!PP>(b, pos, dir, iv, max_t, w);
+        if constexpr (SPLIT) {
+            if (!__any(go)) return false;
+            VRSampler<NFP, REC, MODE> s;
+            s.data = im.pool + b.data_off;
+            s.mask = (b.mask_off >= 0) ? im.masks + b.mask_off : nullptr;
+            s.b = brick_reg(b);
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                s.pa[i] = PP ? dir[i] * b.idds[i] : uni_d(dir[i] * b.idds[i]);
+                s.pb[i] = (pos[i] - b.le[i]) * b.idds[i];
+                s.paf[i] = (float)s.pa[i];
+            }
+            s.tf = &tfc;
+            s.lt = lt;
+            s.nb = nb;
+            s.tform = tform;
+            s.inv_ns = im.inv_ns;
+            s.n_samples = im.n_samples;
+            s.rec = &rec;
+            if (!go) w.cur[0] = w.cur[1] = w.cur[2] = 0;  // (no say in the fast walk's conditions)
+            const VertexFast vf = vertex_fast(s.b, w);
+            if (vf.ok) {
+                walk_vr_ctf_split<(MODE & 2) ? 10 : 0, !PP>(w, go, max_t, s, brick_rsrc(s.data, vf.bytes), vf.k0, vf.k1,
+                                                            s.mask, tfc, lt, seg, lane, wbuf, *par, st[0]);
+            } else if (go) {
+                // every wave walks for its own channel
+#pragma unroll
+                for (int c = 0; c < 4; c++) s.st[c] = st[0];
+                walk_loop(b, w, max_t, s);
+                st[0] = seg == 0 ? s.st[0] : (seg == 1 ? s.st[1] : s.st[2]);
+            }
+            return false;
+        }
         if (go) {
             rec.brick = bid;
             if (KIND == 0) {
@@ -1575,6 +1796,10 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
         if (done) break;
     }
     if (!active) return;
+    if constexpr (SPLIT) {
+        if (seg < 3) im.out[seg * npix + pix] = (float)(1.0 - st[0]);
+        return;
+    }
     if (KIND == 0) {
 #pragma unroll
         for (int f = 0; f < NFP; f++)
@@ -1720,6 +1945,62 @@ void k_persist(const DImg *__restrict__ imgs,
         // 1.1x its time).
         if ((taken++ & 15) == 15 && uni((int)stop_requested(im.stop))) break;
         for (int t = 0; t < cnt; t++) render_tile<KIND, NFP, REC, MODE>(im, tile + t, lane, s_tf + im.tf_slot, wbuf, wave_words);
+    }
+}
+
+// k_persist for volume renders of few tiles (one field, ColorTransferFunction
+// in transmittance form): a workgroup of NSEG waves takes one tile at a time
+// (walk_vr_ctf_split).  A ray's visits are one serial chain, 1.3 us a visit of
+// 10 sub-samples for a lone wave, and with a wave per tile the longest
+// chains are the launch's time while the chip is not full (split_kernel).
+// Here a wave samples a quarter of the visits and steps over the others, at
+// 20 of 270 operations each; the rounds' exchange costs 6 operations a visit.
+// One wave a tile -> four, same images: 256^3 at 200^2 0.63 -> 0.32 ms,
+// perspective 160^3 at 501x333 0.45 -> 0.36, at 200^2 0.44 -> 0.23.
+// Measured and not kept: parts of a ray's chain multiplied together (faster,
+// 0.32 ms for the perspective render, but some pixels one rounding off);
+// the next visit's corners loaded before the present one is sampled, with a
+// wave per tile (no faster: a lone wave waits for its own arithmetic and the
+// table reads, not for the corners).  4 waves per SIMD; 5 spill (0.41 ms).
+template <int MODE>
+__global__ __launch_bounds__(64 * NSEG) __attribute__((amdgpu_waves_per_eu(4)))
+void k_split(const DImg *__restrict__ imgs, const int2 *__restrict__ items, unsigned int *__restrict__ counter,
+             const float4 *__restrict__ tf_all, int tf_bins, int)
+{
+    extern __shared__ float4 s_tf[];
+    __shared__ int2 s_item;
+    for (int i = threadIdx.x; i < tf_bins; i += blockDim.x) s_tf[i] = tf_all[i];
+    const int lane = threadIdx.x & 63, seg = uni((int)(threadIdx.x >> 6));
+    float *qbuf = (float *)(s_tf + tf_bins);
+    // (thread 0's; the queue is k_persist's, by workgroups instead of waves)
+    int part = (int)(blockIdx.x % QSPLIT), left = QSPLIT;
+    int taken = (int)(blockIdx.x & 15);
+    int par = 0;
+    while (true) {
+        if (threadIdx.x == 0) {
+            int2 w = make_int2(-1, 0);
+            while (left > 0) {
+                const unsigned int it = atomicAdd(counter + part * QSTRIDE, 1u);
+                const unsigned int lo = counter[part * QSTRIDE + QLO], hi = counter[part * QSTRIDE + QHI];
+                if (it < hi - lo) {
+                    w = items[lo + it];
+                    break;
+                }
+                left--;
+                part = (part + 1 == QSPLIT) ? 0 : part + 1;
+            }
+            if (w.x >= 0 && (taken++ & 15) == 15 && stop_requested(imgs[w.x].stop)) w.x = -1;
+            s_item = w;
+        }
+        __syncthreads();
+        const int img = uni(s_item.x), tword = uni(s_item.y);
+        if (img < 0) break;
+        const int tile = tword & 0xffffff;
+        const int cnt = max(1, tword >> 24);
+        const DImg &im = imgs[img];
+        for (int t = 0; t < cnt; t++)
+            render_tile<1, 1, false, MODE, true>(im, tile + t, lane, s_tf + im.tf_slot, qbuf, 0, seg, &par);
+        __syncthreads();  // every wave has read the item
     }
 }
 

@@ -32,4 +32,7 @@ kfn_t pick_kernel_vr_d(int nfp, bool rec, int mode);
 pfn_t pick_persist_vr_e(int nfp, bool rec, int mode);
 kfn_t pick_kernel_vr_e(int nfp, bool rec, int mode);
 
+// k_split<kind, mode>, or nullptr where it is not built.
+pfn_t pick_split(int kind, int mode);
+
 }  // namespace ytrc
