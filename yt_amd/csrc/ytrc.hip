@@ -528,11 +528,17 @@ struct DeviceBlocks {
         }
         return e;
     }
+    // (the longest kept go first: a program's present sizes stay)
     void put(char *p, size_t cap)
     {
-        if (cap > KEPT_BLOCK || held + cap > KEPT_TOTAL || kept.size() >= KEPT_COUNT) {
+        if (cap > KEPT_BLOCK) {
             hipFree(p);
             return;
+        }
+        while (!kept.empty() && (held + cap > KEPT_TOTAL || kept.size() >= KEPT_COUNT)) {
+            hipFree(kept.front().first);
+            held -= kept.front().second;
+            kept.erase(kept.begin());
         }
         kept.push_back({p, cap});
         held += cap;
