@@ -394,8 +394,8 @@ pfn_t split_kernel(int n_cu, int kind, int nfp, bool rec, int mode, int n_order,
     const double most = n_order == 1 ? 1.25 : 0.75;
     return chains <= most * 4.0 * n_cu ? pick_split(kind, mode) : nullptr;
 }
-// LDS of k_split after its tables: two rounds' opacities, and the item.
-constexpr size_t SPLIT_LDS = sizeof(float) * SPLIT_Q + 16;
+// LDS of k_split after its tables: two rounds' opacities and lanes, and the item.
+constexpr size_t SPLIT_LDS = sizeof(float) * SPLIT_Q + sizeof(uint64_t) * SPLIT_TOOK + 16;
 
 // Words of LDS per wave that a persistent launch gives after its tables
 // (k_persist's wave_words): the vertex-block buffer with mode bit 4, a

@@ -147,6 +147,12 @@ __device__ __forceinline__ double uni_d(double v)
     const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
+// This lane's bit of a mask that is equal in every lane.
+__device__ __forceinline__ bool lane_bit(uint64_t m)
+{
+    const uint64_t lo = (unsigned)uni((int)(unsigned)m), hi = (unsigned)uni((int)(unsigned)(m >> 32));
+    return __builtin_amdgcn_inverse_ballot_w64((hi << 32) | lo);
+}
 __device__ __forceinline__ double y_fmax(double a, double b) { return (a > b) ? a : b; }
 
 // The host's stop request for a launch (ytrc_batch_cancel), read from

@@ -1204,18 +1204,23 @@ __device__ __forceinline__ VertexFast vertex_fast(const BrickReg &b, const Walk 
 // Waves that share a tile in k_split, visits of a round that each of them
 // samples, and the visits of a round.
 constexpr int NSEG = 4, SPLIT_B = 4, SPLIT_R = NSEG * SPLIT_B;
-// LDS floats of k_split after its tables: two rounds' opacities.
+// LDS of k_split after its tables: two rounds' opacities (floats), then for
+// each of their visits the lanes that it counts for (one bit a lane).
 constexpr int SPLIT_Q = 2 * SPLIT_R * 3 * 64;
+constexpr int SPLIT_TOOK = 2 * SPLIT_R;
 
 // A brick's walk by the NSEG waves of a workgroup, all on the same rays: in
 // each round of SPLIT_R visits wave `seg` samples SPLIT_B and steps over the
 // others, the visits' opacities meet in LDS (qbuf, two rounds in turn, `par`
 // the present one), and waves 0, 1 and 2 take one channel's transmittance T
 // through them in the order of the visits: the FP64 products are those of
-// one wave's walk, in its order, so the same image bit for bit.  A lane past
-// its end leaves opacity 0, which changes no T.  Every wave of the workgroup
-// calls it with the same rays, whose steps do not depend on what it samples,
-// so all of them take the same rounds and meet the same barriers.
+// one wave's walk, in its order, so the same image bit for bit.  T is
+// multiplied only in lanes that the visit counts for (not past their end, the
+// cell unmasked, the value normal), as in one wave's walk: an opacity of 0 in
+// its place would turn an infinite T, an infinite background pixel, into NaN.
+// Every wave of the workgroup calls it with the same rays, whose steps do not
+// depend on what it samples, so all of them take the same rounds and meet the
+// same barriers.
 // SHARED: one direction, walk_vr_ctf_fast's arithmetic; else VRSampler's.
 template <int NS, bool SHARED, class S>
 __device__ __forceinline__ void walk_vr_ctf_split(Walk &w, bool live, double max_t, const S &smp,
@@ -1257,6 +1262,7 @@ __device__ __forceinline__ void walk_vr_ctf_split(Walk &w, bool live, double max
     const float idb = tf.idbin, qc1 = tf.qc1;
     const unsigned D0 = (unsigned)b.d0, D1 = (unsigned)b.d1, D2 = (unsigned)b.d2;
     const int ns = smp.n_samples;
+    uint64_t *took = (uint64_t *)(qbuf + SPLIT_Q);
     int v = 0;  // of the round
     while (__any(live)) {
         // one visit: sampled by this wave or stepped over
@@ -1268,6 +1274,7 @@ __device__ __forceinline__ void walk_vr_ctf_split(Walk &w, bool live, double max
         const bool ge = tm >= max_t;
         if (mine) {
             float Q[3] = {0.0f, 0.0f, 0.0f};
+            bool fine = false;
             if (live) {
                 const double ex = min_f64(tm, max_t);
                 const unsigned o = __umul24((unsigned)c0 >> 2, K0) +
@@ -1327,7 +1334,7 @@ __device__ __forceinline__ void walk_vr_ctf_split(Walk &w, bool live, double max
                     // (quad_visit_ok takes the coefficients as they are)
                     if (!quad_visit_ok(k)) mval = 0;
                 }
-                bool fine = mval == 1;
+                fine = mval == 1;
                 if constexpr (SHARED) {
                     const float mm = __builtin_fabsf(k0) + __builtin_fabsf(ku[1]) + __builtin_fabsf(ku[2]) +
                                      __builtin_fabsf(ku[3]);
@@ -1339,6 +1346,8 @@ __device__ __forceinline__ void walk_vr_ctf_split(Walk &w, bool live, double max
             q[0] = Q[0];
             q[64] = Q[1];
             q[128] = Q[2];
+            const uint64_t counts = __ballot(fine);
+            if (lane == 0) took[par * SPLIT_R + v] = counts;
         }
         if (live) {
             bool out;
@@ -1371,7 +1380,10 @@ __device__ __forceinline__ void walk_vr_ctf_split(Walk &w, bool live, double max
             __syncthreads();
             if (seg < 3) {
                 const float *q = qbuf + par * SPLIT_R * 192 + seg * 64 + lane;
-                for (int i = 0; i < v; i++) T = __builtin_fma(-T, (double)q[i * 192], T);
+                for (int i = 0; i < v; i++) {
+                    const double t = __builtin_fma(-T, (double)q[i * 192], T);
+                    T = lane_bit(took[par * SPLIT_R + i]) ? t : T;
+                }
             }
             par ^= 1;
             v = 0;
