@@ -311,6 +311,9 @@ int ytrc_batch_bytes(const ytrc_batch *b, uint64_t *bytes);
  * stages in LDS (max_tf_bytes); set by the batch flags (YTRC_BATCH_TF_LDS_*).
  * No counterpart in the reference, which has no launches. */
 int ytrc_batch_launch_plan(const ytrc_batch *b, int32_t *n_launches, uint64_t *max_tf_bytes);
+/* Waves that share a ray tile of request i in the batch's launches: 1, or 4
+ * where the batch has few tiles. */
+int ytrc_batch_tile_waves(const ytrc_batch *b, int32_t i, int32_t *waves);
 void ytrc_batch_destroy(ytrc_batch *b);
 
 /* Serving: continuous batching against resident datasets.  The reference

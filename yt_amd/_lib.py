@@ -64,6 +64,7 @@ EXPORTED = [
     "ytrc_batch_set_launch",
     "ytrc_batch_bytes",
     "ytrc_batch_launch_plan",
+    "ytrc_batch_tile_waves",
     "ytrc_batch_destroy",
     "ytrc_batch_kernel_ms",
     "ytrc_batch_request_ms",
@@ -243,6 +244,7 @@ def _declare(lib):
         P, C.c_int32, C.POINTER(C.c_int64), C.POINTER(C.c_uint64), C.POINTER(C.c_int64)]
     lib.ytrc_batch_set_launch.argtypes = [P, C.c_int32, C.c_int32]
     lib.ytrc_batch_bytes.argtypes = [P, C.POINTER(C.c_uint64)]
+    lib.ytrc_batch_tile_waves.argtypes = [P, C.c_int32, C.POINTER(C.c_int32)]
     lib.ytrc_batch_launch_plan.argtypes = [P, C.POINTER(C.c_int32), C.POINTER(C.c_uint64)]
     lib.ytrc_batch_destroy.argtypes = [P]
     lib.ytrc_batch_destroy.restype = None
@@ -742,6 +744,13 @@ class Batch:
         n, b = C.c_int32(), C.c_uint64()
         _check(lib().ytrc_batch_launch_plan(self._h, C.byref(n), C.byref(b)))
         return n.value, b.value
+
+    def tile_waves(self, i):
+        """Waves that share a ray tile of request i: 1, or 4 where the batch
+        has few tiles."""
+        n = C.c_int32()
+        _check(lib().ytrc_batch_tile_waves(self._h, int(i), C.byref(n)))
+        return n.value
 
     def read_image(self, i):
         nv = self.specs[i].nv

@@ -394,8 +394,6 @@ pfn_t split_kernel(int n_cu, int kind, int nfp, bool rec, int mode, int n_order,
     const double most = n_order == 1 ? 1.25 : 0.75;
     return chains <= most * 4.0 * n_cu ? pick_split(kind, mode) : nullptr;
 }
-// LDS of k_split after its tables: two rounds' opacities and lanes, and the item.
-constexpr size_t SPLIT_LDS = sizeof(float) * SPLIT_Q + sizeof(uint64_t) * SPLIT_TOOK + 16;
 
 // Words of LDS per wave that a persistent launch gives after its tables
 // (k_persist's wave_words): the vertex-block buffer with mode bit 4, a
@@ -627,6 +625,7 @@ struct ytrc_batch {
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;  // persistent: the second stream's fork and join
     std::vector<hipEvent_t> ev_req;  // plain mode: before/after each request
     std::vector<PGroup> groups;      // persistent mode
+    std::vector<int> group_of;       // and each request's
     unsigned int *counters = nullptr;
     const float4 *tf_all = nullptr;
     int tf_bins = 0;
@@ -751,6 +750,12 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 }  // namespace
 
 namespace {
+
+// Whether a launch of a persistent batch takes four waves to a tile.
+bool split_launch(const ytrc_batch *b, const PGroup &g)
+{
+    return g.split != nullptr && b->waves_per_group == NSEG;
+}
 
 // Gives a batch's stop flag back (ctx->mu held).
 void release_stop(ytrc_batch *b)
@@ -1812,6 +1817,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     B->ctx = ctx;
     B->flags = batch_flags;
     B->reqs.resize(n_req);
+    B->group_of.resize(n_req);
     B->h_imgs.resize(n_req);
     for (int i = 0; i < n_req; i++) B->reqs[i] = P[i].q;
     auto bad = [&](int code, const std::string &m) {
@@ -2006,6 +2012,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
                 g.split = split_kernel(ctx->n_cu, g.kind, g.nfp, g.rec, g.mode, P[i].q.r.n_order, chains_all);
         g.n_items = (int)items.size();
         g.counter = (int)B->groups.size();
+        for (int i : ids) B->group_of[(size_t)i] = g.counter;
         g.tf_base = plan_base[L];
         g.tf_bins = plan_bins[L];
         g.lds = has_tf(g.kind) ? sizeof(float4) * (size_t)g.tf_bins : 0;
@@ -2129,6 +2136,14 @@ int ytrc_batch_launch_plan(const ytrc_batch *b, int32_t *n_launches, uint64_t *m
     return YTRC_OK;
 }
 
+int ytrc_batch_tile_waves(const ytrc_batch *b, int32_t i, int32_t *waves)
+{
+    if (b == nullptr || waves == nullptr) return fail(YTRC_EINVAL, "ytrc_batch_tile_waves: NULL argument");
+    if (i < 0 || i >= (int)b->reqs.size()) return fail(YTRC_EINVAL, "ytrc_batch_tile_waves: bad index");
+    *waves = (b->flags & YTRC_BATCH_PERSISTENT) && split_launch(b, b->groups[(size_t)b->group_of[(size_t)i]]) ? NSEG : 1;
+    return YTRC_OK;
+}
+
 int ytrc_batch_set_launch(ytrc_batch *b, int32_t waves_per_group, int32_t groups_per_cu)
 {
     if (b == nullptr) return fail(YTRC_EINVAL, "ytrc_batch_set_launch: NULL batch");
@@ -2179,7 +2194,7 @@ int enqueue_persistent(ytrc_batch *b, hipStream_t s)
         PGroup &g = b->groups[order[k]];
         hipStream_t gs = (k == 0) ? s : b->ctx->stream2;
         // each wave's buffer after the tables
-        const bool split = g.split != nullptr && b->waves_per_group == NSEG;
+        const bool split = split_launch(b, g);
         const pfn_t fn = split ? g.split : g.fn;
         const int ww = split ? 0 : required_wave_words(g.kind, g.nfp, g.rec, g.mode);
         const size_t lds = g.lds + (split ? SPLIT_LDS : (size_t)b->waves_per_group * ww * sizeof(unsigned));

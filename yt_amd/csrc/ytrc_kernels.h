@@ -1205,9 +1205,12 @@ __device__ __forceinline__ VertexFast vertex_fast(const BrickReg &b, const Walk 
 // samples, and the visits of a round.
 constexpr int NSEG = 4, SPLIT_B = 4, SPLIT_R = NSEG * SPLIT_B;
 // LDS of k_split after its tables: two rounds' opacities (floats), then for
-// each of their visits the lanes that it counts for (one bit a lane).
+// each of their visits the lanes that it counts for (one bit a lane), then
+// the workgroup's item.  All of it is the launch's dynamic LDS, so that the
+// host's SPLIT_LDS is all the kernel takes after its tables.
 constexpr int SPLIT_Q = 2 * SPLIT_R * 3 * 64;
 constexpr int SPLIT_TOOK = 2 * SPLIT_R;
+constexpr int SPLIT_LDS = SPLIT_Q * 4 + SPLIT_TOOK * 8 + 16;
 
 // A brick's walk by the NSEG waves of a workgroup, all on the same rays: in
 // each round of SPLIT_R visits wave `seg` samples SPLIT_B and steps over the
@@ -1980,10 +1983,10 @@ void k_split(const DImg *__restrict__ imgs, const int2 *__restrict__ items, unsi
              const float4 *__restrict__ tf_all, int tf_bins, int)
 {
     extern __shared__ float4 s_tf[];
-    __shared__ int2 s_item;
     for (int i = threadIdx.x; i < tf_bins; i += blockDim.x) s_tf[i] = tf_all[i];
     const int lane = threadIdx.x & 63, seg = uni((int)(threadIdx.x >> 6));
     float *qbuf = (float *)(s_tf + tf_bins);
+    int2 *s_item = (int2 *)((uint64_t *)(qbuf + SPLIT_Q) + SPLIT_TOOK);
     // (thread 0's; the queue is k_persist's, by workgroups instead of waves)
     int part = (int)(blockIdx.x % QSPLIT), left = QSPLIT;
     int taken = (int)(blockIdx.x & 15);
@@ -2002,10 +2005,10 @@ void k_split(const DImg *__restrict__ imgs, const int2 *__restrict__ items, unsi
                 part = (part + 1 == QSPLIT) ? 0 : part + 1;
             }
             if (w.x >= 0 && (taken++ & 15) == 15 && stop_requested(imgs[w.x].stop)) w.x = -1;
-            s_item = w;
+            *s_item = w;
         }
         __syncthreads();
-        const int img = uni(s_item.x), tword = uni(s_item.y);
+        const int img = uni(s_item->x), tword = uni(s_item->y);
         if (img < 0) break;
         const int tile = tword & 0xffffff;
         const int cnt = max(1, tword >> 24);
