@@ -103,7 +103,9 @@ typedef struct ytrc_ctx ytrc_ctx;
 typedef struct ytrc_batch ytrc_batch;
 
 /* Context: one per device.  budget_bytes caps the device memory this context
- * may hold (datasets + batches); 0 means no cap. */
+ * may hold (datasets, batches, servers, and freed blocks of them that it keeps
+ * for its next calls); 0 means no cap.  Kept blocks are given back before
+ * anything is refused for them. */
 int ytrc_ctx_create(int32_t device, uint64_t budget_bytes, ytrc_ctx **out);
 void ytrc_ctx_destroy(ytrc_ctx *ctx);
 int ytrc_ctx_used_bytes(const ytrc_ctx *ctx, uint64_t *used, uint64_t *budget);
@@ -177,7 +179,8 @@ int ytrc_dataset_build_vr(ytrc_ctx *ctx, int32_t n_grids, const ytrc_grid_desc *
  * brick preparation against the host's. */
 int ytrc_dataset_read_points(ytrc_ctx *ctx, int32_t ds_id, int32_t brick, float *out, int64_t cap,
                              int64_t *n_out);
-/* Frees a dataset's device memory.  Refused with YTRC_EBUSY while a live
+/* Frees a dataset's device memory (a context keeps freed blocks of up to 32
+ * MiB, 96 MiB in all, for its next calls).  Refused with YTRC_EBUSY while a live
  * batch or an unread server request uses it (a batch holds its datasets
  * until ytrc_batch_destroy; a server request until it is read, cancelled or
  * the server is destroyed). */

@@ -33,6 +33,7 @@
 #include "ytrc_device.h"
 #include "ytrc_host.h"
 #include "ytrc_kernels.h"
+#include "ytrc_memory.h"
 #include "ytrc_pick.h"
 #include "ytrc_transfer.h"
 
@@ -482,75 +483,13 @@ constexpr size_t PIN_BYTES = 2u << 20;
 constexpr size_t PIN_OUT = 4u << 20;
 constexpr int STOPS = 64, STOP_STRIDE = 16;
 
-// Device memory of dataset pools, batches and staged fields: freed blocks of
-// up to KEPT_BLOCK bytes are kept for the next one, KEPT_TOTAL in all.  A
-// program that renders frame after frame makes and frees the same blocks, and
-// an hipMalloc of 10 MB took up to 0.47 ms, an hipFree 0.07 ms, beside kernels
-// of 0.1 to 0.3 ms.  Used with ctx->mu held; a block is put back only when
-// nothing on the device uses it any more.
-struct DeviceBlocks {
-    static constexpr size_t KEPT_BLOCK = 32u << 20, KEPT_TOTAL = 96u << 20, KEPT_COUNT = 8;
-    std::vector<std::pair<char *, size_t>> kept;
-    size_t held = 0;
-
-    ~DeviceBlocks() { clear(); }
-    void clear()
-    {
-        for (auto &b : kept) hipFree(b.first);
-        kept.clear();
-        held = 0;
-    }
-    // A block of at least `bytes`: the smallest kept one that is no more than
-    // twice as large, else a new one.
-    hipError_t get(size_t bytes, char **p, size_t *cap)
-    {
-        int at = -1;
-        for (int i = 0; i < (int)kept.size(); i++) {
-            const size_t c = kept[(size_t)i].second;
-            if (c >= bytes && c / 2 <= bytes && (at < 0 || c < kept[(size_t)at].second)) at = i;
-        }
-        if (at >= 0) {
-            *p = kept[(size_t)at].first;
-            *cap = kept[(size_t)at].second;
-            held -= *cap;
-            kept.erase(kept.begin() + at);
-            return hipSuccess;
-        }
-        *p = nullptr;
-        *cap = bytes;
-        hipError_t e = hipMalloc((void **)p, bytes);
-        if (e == hipErrorOutOfMemory && !kept.empty()) {
-            (void)hipGetLastError();
-            clear();
-            e = hipMalloc((void **)p, bytes);
-        }
-        return e;
-    }
-    // (the longest kept go first: a program's present sizes stay)
-    void put(char *p, size_t cap)
-    {
-        if (cap > KEPT_BLOCK) {
-            hipFree(p);
-            return;
-        }
-        while (!kept.empty() && (held + cap > KEPT_TOTAL || kept.size() >= KEPT_COUNT)) {
-            hipFree(kept.front().first);
-            held -= kept.front().second;
-            kept.erase(kept.begin());
-        }
-        kept.push_back({p, cap});
-        held += cap;
-    }
-};
-
 struct ytrc_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     // a second stream (default priority) for the concurrent launches of a
     // persistent batch, joined back to `stream` by the batch's events
     hipStream_t stream2 = nullptr;
-    uint64_t budget = 0;
-    uint64_t used = 0;
+    DeviceMemory mem;
     int n_cu = 0;
     size_t max_lds = 64 * 1024;  // LDS bytes one workgroup may allocate
     std::string name;            // marketing name and ISA of the device
@@ -558,7 +497,6 @@ struct ytrc_ctx {
     char *scratch = nullptr;     // this device's `scratch` array (ytrc_render_noalloc)
     std::mutex *scratch_mu = nullptr;  // serialises the calls that share it
     Transfer xfer;               // images to and fields from the caller's memory
-    DeviceBlocks blocks;
     // Batches' stop flags, a line each in one page of pinned memory (an
     // hipHostMalloc and its hipHostFree took 0.08 ms); those out of use.
     int *stops = nullptr;
@@ -825,14 +763,14 @@ int dataset_alloc(ytrc_ctx *ctx, const char *who, int n_bricks, const ytrc_brick
     }
     const uint64_t bytes = (uint64_t)pool_floats * 4 + (uint64_t)mask_bytes +
                            (uint64_t)n_bricks * sizeof(DBrick);
-    if (ctx->budget != 0 && ctx->used + bytes > ctx->budget)
+    if (!ctx->mem.fits(bytes))
         return fail(YTRC_EBUDGET, w + ": " + std::to_string(bytes) + " bytes exceed the HBM budget");
     auto dev = [&](hipError_t e, const char *what) {
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, w + ": " + what + ": " + hipGetErrorString(e));
     };
     char *pool = nullptr;
-    hipError_t e = ctx->blocks.get((size_t)pool_floats * 4, &pool, &ds.pool_cap);
+    hipError_t e = ctx->mem.get((size_t)pool_floats * 4, bytes, &pool, &ds.pool_cap);
     if (e != hipSuccess) return dev(e, "hipMalloc(pool)");
     ds.d_pool = (float *)pool;
     if (mask_bytes > 0) {
@@ -857,7 +795,7 @@ int dataset_alloc(ytrc_ctx *ctx, const char *who, int n_bricks, const ytrc_brick
 void dataset_release(ytrc_ctx *ctx, Dataset &ds)
 {
     if (ds.d_bricks) hipFree(ds.d_bricks);
-    if (ds.d_pool) ctx->blocks.put((char *)ds.d_pool, ds.pool_cap);
+    if (ds.d_pool) ctx->mem.put((char *)ds.d_pool, ds.pool_cap);
     if (ds.d_masks) hipFree(ds.d_masks);
     ds.d_bricks = nullptr;
     ds.d_pool = nullptr;
@@ -875,14 +813,15 @@ struct Staging {
     Staging(const Staging &) = delete;
     ~Staging()
     {
-        if (p) ctx->blocks.put(p, cap);
+        if (p) ctx->mem.put(p, cap);
     }
-    hipError_t get(size_t bytes) { return ctx->blocks.get(bytes, &p, &cap); }
+    // `with`: bytes of the dataset that the fields go to
+    hipError_t get(size_t bytes, uint64_t with) { return ctx->mem.get(bytes, with + bytes, &p, &cap); }
 };
 
 int dataset_commit(ytrc_ctx *ctx, Dataset &ds, int32_t *ds_id_out)
 {
-    ctx->used += ds.bytes;
+    ctx->mem.used += ds.bytes;
     const int id = ctx->next_ds++;
     ctx->datasets[id] = std::move(ds);
     *ds_id_out = id;
@@ -934,7 +873,7 @@ int ytrc_ctx_create(int32_t device, uint64_t budget_bytes, ytrc_ctx **out)
     HIPCHK(hipSetDevice(device));
     ytrc_ctx *c = new ytrc_ctx();
     c->device = device;
-    c->budget = budget_bytes;
+    c->mem.budget = budget_bytes;
     hipDeviceProp_t prop;
     hipError_t e = hipGetDeviceProperties(&prop, device);
     if (e != hipSuccess) {
@@ -1010,8 +949,8 @@ int ytrc_ctx_device_name(const ytrc_ctx *ctx, char *buf, int32_t cap)
 int ytrc_ctx_used_bytes(const ytrc_ctx *ctx, uint64_t *used, uint64_t *budget)
 {
     if (ctx == nullptr) return fail(YTRC_EINVAL, "ytrc_ctx_used_bytes: ctx is NULL");
-    if (used) *used = ctx->used;
-    if (budget) *budget = ctx->budget;
+    if (used) *used = ctx->mem.used;
+    if (budget) *budget = ctx->mem.budget;
     return YTRC_OK;
 }
 
@@ -1033,7 +972,7 @@ int ytrc_dataset_upload(ytrc_ctx *ctx, int32_t n_bricks, const ytrc_brick_desc *
     // Each brick field goes to the device in C order as given (float64 or
     // float32) and k_store_field converts it to float32 in the device
     // layout, fields interleaved per point.  Fields are staged together, up
-    // to STAGE_MOST bytes or one field at a time; copies and kernels are
+    // to STAGE_MOST bytes and what a budget leaves, or one field at a time; copies and kernels are
     // ordered on the stream.
     constexpr size_t STAGE_MOST = 32u << 20;
     const size_t esz = src_dtype == 0 ? 8 : 4;
@@ -1046,9 +985,9 @@ int ytrc_dataset_upload(ytrc_ctx *ctx, int32_t n_bricks, const ytrc_brick_desc *
         most = std::max(most, points(b) * esz);
         total += points(b) * esz * (size_t)n_fields;
     }
-    const size_t room = std::max(most, std::min(total, STAGE_MOST));
+    const size_t room = std::max<size_t>(most, (size_t)std::min<uint64_t>(std::min(total, STAGE_MOST), ctx->mem.left(ds.bytes)));
     Staging stg(ctx);
-    hipError_t e = stg.get(room);
+    hipError_t e = stg.get(room, ds.bytes);
     if (e != hipSuccess) {
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, std::string("hipMalloc(staging): ") + hipGetErrorString(e));
@@ -1158,7 +1097,7 @@ int ytrc_dataset_build_vr(ytrc_ctx *ctx, int32_t n_grids, const ytrc_grid_desc *
     int rc = dataset_alloc(ctx, who, n_leaves, bd.data(), n_fields, mask_ptrs, ds);
     if (rc != YTRC_OK) return rc;
     Staging stg(ctx);
-    hipError_t e = stg.get((size_t)cells * esz);
+    hipError_t e = stg.get((size_t)cells * esz, ds.bytes);
     if (e != hipSuccess) {
         dataset_release(ctx, ds);
         return fail(YTRC_EDEVICE, std::string("hipMalloc(cells): ") + hipGetErrorString(e));
@@ -1250,7 +1189,7 @@ int ytrc_dataset_free(ytrc_ctx *ctx, int32_t ds_id)
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream2));
-    ctx->used -= it->second.bytes;
+    ctx->mem.used -= it->second.bytes;
     dataset_release(ctx, it->second);
     ctx->datasets.erase(it);
     return YTRC_OK;
@@ -1823,7 +1762,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     auto bad = [&](int code, const std::string &m) {
         if (B->arena) {
             hipFree(B->arena);  // (it may hold copies under way)
-            ctx->used -= B->arena_bytes;
+            ctx->mem.used -= B->arena_bytes;
         }
         release_stop(B);
         if (B->ev0) hipEventDestroy(B->ev0);
@@ -2045,12 +1984,12 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     off = align_up(off + sizeof(unsigned int) * QCOUNTERS * std::max<size_t>(1, B->groups.size()), 256);
     const size_t imgs_off = off;
     off = align_up(off + sizeof(DImg) * n_req, 256);
-    if (ctx->budget != 0 && ctx->used + off > ctx->budget)
+    if (!ctx->mem.fits(off))
         return bad(YTRC_EBUDGET, "ytrc_batch_create: " + std::to_string(off) + " bytes exceed the HBM budget");
-    hipError_t e = ctx->blocks.get(off, &B->arena, &B->arena_cap);
+    hipError_t e = ctx->mem.get(off, off, &B->arena, &B->arena_cap);
     if (e != hipSuccess) return bad(YTRC_EDEVICE, std::string("hipMalloc: ") + hipGetErrorString(e));
     B->arena_bytes = off;
-    ctx->used += off;
+    ctx->mem.used += off;
     char *A = B->arena;
     // The stop flag: fine-grained pinned host memory that the kernels read
     // at system scope once per tile.
@@ -2557,8 +2496,8 @@ void ytrc_batch_destroy(ytrc_batch *b)
     hipStreamSynchronize(b->ctx->stream);
     if (b->arena) {
         std::lock_guard<std::mutex> lk(b->ctx->mu);
-        b->ctx->blocks.put(b->arena, b->arena_cap);
-        b->ctx->used -= b->arena_bytes;
+        b->ctx->mem.used -= b->arena_bytes;
+        b->ctx->mem.put(b->arena, b->arena_cap);
     }
     {
         std::lock_guard<std::mutex> lk(b->ctx->mu);
@@ -3009,8 +2948,9 @@ int ytrc_server_create(ytrc_ctx *ctx, int32_t max_requests, uint64_t budget_byte
     if (budget_bytes < (1u << 20)) return fail(YTRC_EINVAL, "ytrc_server_create: budget below 1 MiB");
     std::lock_guard<std::mutex> lk(ctx->mu);
     HIPCHK(hipSetDevice(ctx->device));
-    if (ctx->budget != 0 && ctx->used + budget_bytes > ctx->budget)
+    if (!ctx->mem.fits(budget_bytes))
         return fail(YTRC_EBUDGET, "ytrc_server_create: server budget exceeds the context budget");
+    ctx->mem.make_room(budget_bytes);
     ytrc_server *S = new ytrc_server();
     S->ctx = ctx;
     S->max_slots = max_requests;
@@ -3055,7 +2995,7 @@ int ytrc_server_create(ytrc_ctx *ctx, int32_t max_requests, uint64_t budget_byte
         if (e != hipSuccess) return bad(e, "hipEventCreate");
     }
     for (int i = max_requests - 1; i >= 0; i--) S->free_slots.push_back(i);
-    ctx->used += budget_bytes;
+    ctx->mem.used += budget_bytes;
     *out = S;
     return YTRC_OK;
 }
@@ -3317,7 +3257,7 @@ void ytrc_server_destroy(ytrc_server *S)
     }
     {
         std::lock_guard<std::mutex> lk(S->ctx->mu);
-        S->ctx->used -= S->budget;
+        S->ctx->mem.used -= S->budget;
         // Requests never read or cancelled give their datasets back.
         for (auto &kv : S->reqs) {
             if (!kv.second.ds_ref) continue;
