@@ -5,6 +5,8 @@ CPU: the header compiled against an allocator that counts what is held.
   it, and what is refused depends only on what is in use, as without kept
   blocks.
 * Without one, at most 96 MiB in 8 blocks of at most 32 MiB are kept.
+* An allocation that finds no room on the device takes every context's kept
+  blocks before it fails, also while other threads get and put blocks.
 """
 
 import os
@@ -20,11 +22,14 @@ HIP = r"""
 #include <cstdint>
 #include <cstdlib>
 #include <map>
+#include <mutex>
 enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2 };
 inline std::map<void *, size_t> g_live;
 inline uint64_t g_held = 0, g_size = UINT64_MAX;  // of the device
+inline std::mutex g_mu;
 inline hipError_t hipMalloc(void **p, size_t n)
 {
+    std::lock_guard<std::mutex> lk(g_mu);
     if (g_held + n > g_size) return hipErrorOutOfMemory;
     *p = malloc(1);
     g_live[*p] = n;
@@ -33,6 +38,7 @@ inline hipError_t hipMalloc(void **p, size_t n)
 }
 inline hipError_t hipFree(void *p)
 {
+    std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_live.find(p);
     if (it == g_live.end()) abort();
     g_held -= it->second;
@@ -110,6 +116,63 @@ int main()
 }
 """
 
+FULL = r"""
+#include <cstdio>
+#include <thread>
+#include "ytrc_memory.h"
+#define CHECK(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
+int main()
+{
+    const size_t MB = 1u << 20;
+    g_size = 100 * MB;
+    {
+        DeviceMemory a, b;
+        struct { char *p; size_t cap; } keep[3];
+        for (int i = 0; i < 3; i++) CHECK((i ? a : b).get(30 * MB, 30 * MB, &keep[i].p, &keep[i].cap) == hipSuccess);
+        for (int i = 0; i < 3; i++) (i ? a : b).put(keep[i].p, keep[i].cap);
+        CHECK(g_held == 90 * MB);
+        // a server's arena, a mask: neither is a kept block
+        float *arena = nullptr;
+        CHECK(DeviceMemory::alloc(&arena, 95 * MB) == hipSuccess);
+        CHECK(g_held == 95 * MB);
+        char *p;
+        size_t cap;
+        CHECK(a.get(6 * MB, 6 * MB, &p, &cap) == hipErrorOutOfMemory);
+        CHECK(b.get(5 * MB, 5 * MB, &p, &cap) == hipSuccess);
+        b.put(p, cap);
+        hipFree(arena);
+        // (one context's blocks for another's)
+        CHECK(a.get(98 * MB, 98 * MB, &p, &cap) == hipSuccess);
+        a.put(p, cap);
+    }
+    CHECK(g_held == 0);
+    std::vector<std::thread> threads;
+    std::atomic<int> bad{0};
+    for (int t = 0; t < 6; t++)
+        threads.emplace_back([&, t] {
+            DeviceMemory m;
+            for (int i = 0; i < 3000; i++) {
+                char *p;
+                size_t cp;
+                // (a block is at most twice as large as asked for: at most
+                // 6 (8 + 4) of 100 MB are out at once)
+                const size_t n = (size_t)(1 + (i * 7 + t) % 4) * MB;
+                if (m.get(n, n, &p, &cp) != hipSuccess) bad++;
+                else {
+                    float *r;
+                    if (DeviceMemory::alloc(&r, 4 * MB) != hipSuccess) bad++;
+                    else hipFree((char *)r);
+                    m.put(p, cp);
+                }
+            }
+        });
+    for (auto &t : threads) t.join();
+    CHECK(g_held == 0 && g_live.empty());
+    puts("ok");
+    return 0;
+}
+"""
+
 
 def _run(tmp_path, source):
     cxx = shutil.which("g++") or shutil.which("c++")
@@ -128,3 +191,7 @@ def _run(tmp_path, source):
 
 def test_kept_blocks_stay_within_the_budget(tmp_path):
     _run(tmp_path, BUDGET)
+
+
+def test_no_allocation_fails_for_kept_blocks(tmp_path):
+    _run(tmp_path, FULL)

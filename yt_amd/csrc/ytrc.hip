@@ -774,10 +774,10 @@ int dataset_alloc(ytrc_ctx *ctx, const char *who, int n_bricks, const ytrc_brick
     if (e != hipSuccess) return dev(e, "hipMalloc(pool)");
     ds.d_pool = (float *)pool;
     if (mask_bytes > 0) {
-        e = hipMalloc(&ds.d_masks, (size_t)mask_bytes);
+        e = DeviceMemory::alloc(&ds.d_masks, (size_t)mask_bytes);
         if (e != hipSuccess) return dev(e, "hipMalloc(masks)");
     }
-    e = hipMalloc(&ds.d_bricks, (size_t)n_bricks * sizeof(DBrick));
+    e = DeviceMemory::alloc(&ds.d_bricks, (size_t)n_bricks * sizeof(DBrick));
     if (e != hipSuccess) return dev(e, "hipMalloc(bricks)");
     for (int b = 0; b < n_bricks; b++) {
         const DBrick &h = ds.h_bricks[b];
@@ -2453,8 +2453,8 @@ int ytrc_hbm_probe(ytrc_ctx *ctx, uint64_t bytes, int32_t iters, float *gbps, fl
     HIPCHK(hipSetDevice(ctx->device));
     const size_t n = (size_t)(bytes / 16);
     float4 *a = nullptr, *b = nullptr;
-    HIPCHK(hipMalloc(&a, n * 16));
-    hipError_t e = hipMalloc(&b, n * 16);
+    HIPCHK(DeviceMemory::alloc(&a, n * 16));
+    hipError_t e = DeviceMemory::alloc(&b, n * 16);
     if (e != hipSuccess) {
         hipFree(a);
         return fail(YTRC_EDEVICE, std::string("hipMalloc: ") + hipGetErrorString(e));
@@ -2971,13 +2971,13 @@ int ytrc_server_create(ytrc_ctx *ctx, int32_t max_requests, uint64_t budget_byte
         delete S;
         return fail(YTRC_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
     };
-    hipError_t e = hipMalloc(&S->arena, budget_bytes);
+    hipError_t e = DeviceMemory::alloc(&S->arena, budget_bytes);
     if (e != hipSuccess) return bad(e, "hipMalloc(arena)");
     S->alloc.init(S->arena, budget_bytes);
-    e = hipMalloc(&S->d_slots, sizeof(DImg) * max_requests);
+    e = DeviceMemory::alloc(&S->d_slots, sizeof(DImg) * max_requests);
     if (e != hipSuccess) return bad(e, "hipMalloc(slots)");
     S->tf_cap = (int)(ctx->max_lds / sizeof(float4));
-    e = hipMalloc(&S->d_tf, sizeof(float4) * S->tf_cap);
+    e = DeviceMemory::alloc(&S->d_tf, sizeof(float4) * S->tf_cap);
     if (e != hipSuccess) return bad(e, "hipMalloc(tf)");
     for (auto &c : S->chunks) {
         // (k_stage moves whole 16-byte units)
@@ -2985,9 +2985,9 @@ int ytrc_server_create(ytrc_ctx *ctx, int32_t max_requests, uint64_t budget_byte
         if (e != hipSuccess) return bad(e, "hipHostMalloc(items)");
         e = hipHostMalloc((void **)&c.h_stage, SRV_STAGE_BYTES, hipHostMallocDefault);
         if (e != hipSuccess) return bad(e, "hipHostMalloc(staging)");
-        e = hipMalloc(&c.d_items, sizeof(int2) * (chunk_tiles + 1));
+        e = DeviceMemory::alloc(&c.d_items, sizeof(int2) * (chunk_tiles + 1));
         if (e != hipSuccess) return bad(e, "hipMalloc(items)");
-        e = hipMalloc(&c.d_counters, sizeof(unsigned int) * SRV_MAX_VARIANTS * QCOUNTERS);
+        e = DeviceMemory::alloc(&c.d_counters, sizeof(unsigned int) * SRV_MAX_VARIANTS * QCOUNTERS);
         if (e != hipSuccess) return bad(e, "hipMalloc(counters)");
         e = hipEventCreateWithFlags(&c.done, hipEventDisableTiming);
         if (e != hipSuccess) return bad(e, "hipEventCreate");

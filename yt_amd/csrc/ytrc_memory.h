@@ -3,8 +3,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
+#include <set>
 #include <utility>
 #include <vector>
 
@@ -17,6 +20,10 @@ namespace {
 // of 0.1 to 0.3 ms.  Used with ctx->mu held; a block is put back only when
 // nothing on the device uses it any more.
 //
+// No allocation fails for the sake of kept blocks: where the device has no
+// room, every context of it gives its blocks back and the allocation is tried
+// again (alloc).
+//
 // With a budget, what the context holds stays within it: datasets, batches
 // and servers (`used`) and the kept blocks together.  Kept blocks never make
 // it refuse anything: they are given back first.  They serve only blocks of
@@ -27,7 +34,22 @@ struct DeviceMemory {
     uint64_t budget = 0;  // 0: none
     uint64_t used = 0;    // bytes of datasets, batches and servers
 
-    ~DeviceMemory() { clear(); }
+    DeviceMemory()
+    {
+        All &all = everyone();
+        std::lock_guard<std::mutex> lk(all.mu);
+        all.set.insert(this);
+    }
+    DeviceMemory(const DeviceMemory &) = delete;
+    ~DeviceMemory()
+    {
+        {
+            All &all = everyone();
+            std::lock_guard<std::mutex> lk(all.mu);
+            all.set.erase(this);
+        }
+        clear();
+    }
 
     // Whether `bytes` more may be used.
     bool fits(uint64_t bytes) const { return budget == 0 || used + bytes <= budget; }
@@ -40,39 +62,51 @@ struct DeviceMemory {
     // kept go first: a program's present sizes stay.
     void make_room(uint64_t more)
     {
-        const uint64_t most = left(more);
-        while (!kept.empty() && held > most) drop();
+        std::lock_guard<std::mutex> lk(mu);
+        drop_above(left(more));
+    }
+    // hipMalloc; where the device has no room, once more without any
+    // context's kept blocks.
+    template <class T>
+    static hipError_t alloc(T **p, size_t bytes)
+    {
+        hipError_t e = hipMalloc((void **)p, bytes);
+        if (e != hipErrorOutOfMemory) return e;
+        (void)hipGetLastError();
+        All &all = everyone();
+        std::lock_guard<std::mutex> lk(all.mu);
+        all.full = true;  // (a block put back meanwhile is not kept)
+        for (DeviceMemory *m : all.set) m->clear();
+        e = hipMalloc((void **)p, bytes);
+        all.full = false;
+        return e;
     }
     // A block of at least `bytes`, one of the `more` bytes that the caller is
     // about to use: the smallest kept one that is no more than twice as large
     // (with a budget: of that size), else a new one.
     hipError_t get(size_t bytes, uint64_t more, char **p, size_t *cap)
     {
-        int at = -1;
-        for (int i = 0; i < (int)kept.size(); i++) {
-            const size_t c = kept[(size_t)i].second;
-            if (c >= bytes && (budget == 0 ? c / 2 <= bytes : c == bytes) &&
-                (at < 0 || c < kept[(size_t)at].second))
-                at = i;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            int at = -1;
+            for (int i = 0; i < (int)kept.size(); i++) {
+                const size_t c = kept[(size_t)i].second;
+                if (c >= bytes && (budget == 0 ? c / 2 <= bytes : c == bytes) &&
+                    (at < 0 || c < kept[(size_t)at].second))
+                    at = i;
+            }
+            if (at >= 0) {
+                *p = kept[(size_t)at].first;
+                *cap = kept[(size_t)at].second;
+                held -= *cap;
+                kept.erase(kept.begin() + at);
+            }
+            drop_above(left(more));
+            if (at >= 0) return hipSuccess;
         }
-        if (at >= 0) {
-            *p = kept[(size_t)at].first;
-            *cap = kept[(size_t)at].second;
-            held -= *cap;
-            kept.erase(kept.begin() + at);
-            make_room(more);
-            return hipSuccess;
-        }
-        make_room(more);
         *p = nullptr;
         *cap = bytes;
-        hipError_t e = hipMalloc((void **)p, bytes);
-        if (e == hipErrorOutOfMemory && !kept.empty()) {
-            (void)hipGetLastError();
-            clear();
-            e = hipMalloc((void **)p, bytes);
-        }
-        return e;
+        return alloc(p, bytes);
     }
     // Gives a block back; its bytes are no longer among `used`.
     void put(char *p, size_t cap)
@@ -81,15 +115,33 @@ struct DeviceMemory {
             hipFree(p);
             return;
         }
+        std::lock_guard<std::mutex> lk(mu);
+        if (everyone().full) {
+            hipFree(p);
+            return;
+        }
         while (!kept.empty() && (held + cap > KEPT_TOTAL || kept.size() >= KEPT_COUNT)) drop();
         kept.push_back({p, cap});
         held += cap;
-        make_room(0);
+        drop_above(left(0));
     }
 
   private:
+    std::mutex mu;  // of the kept blocks: another context's thread may clear them
     std::vector<std::pair<char *, size_t>> kept;
     size_t held = 0;
+
+    struct All {
+        std::mutex mu;
+        std::set<DeviceMemory *> set;
+        std::atomic<bool> full{false};
+    };
+    // (never destroyed: a context may outlive static objects)
+    static All &everyone()
+    {
+        static All *all = new All();
+        return *all;
+    }
 
     void drop()
     {
@@ -97,9 +149,14 @@ struct DeviceMemory {
         held -= kept.front().second;
         kept.erase(kept.begin());
     }
+    void drop_above(uint64_t most)
+    {
+        while (!kept.empty() && held > most) drop();
+    }
     void clear()
     {
-        while (!kept.empty()) drop();
+        std::lock_guard<std::mutex> lk(mu);
+        drop_above(0);
     }
 };
 
