@@ -2125,6 +2125,17 @@ int enqueue_persistent(ytrc_batch *b, hipStream_t s)
     };
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return work(x) > work(y); });
     const bool fork = order.size() >= 2;
+    // Where a launch fails, those on the second stream are waited for: the
+    // batch's memory may serve another as soon as the first stream is idle
+    // (ytrc_batch_destroy).
+    struct Unjoined {
+        hipStream_t s2;
+        bool armed;
+        ~Unjoined()
+        {
+            if (armed) (void)hipStreamSynchronize(s2);
+        }
+    } unjoined{b->ctx->stream2, fork};
     if (fork) {
         HIPCHK(hipEventRecord(b->ev_fork, s));
         HIPCHK(hipStreamWaitEvent(b->ctx->stream2, b->ev_fork, 0));
@@ -2155,6 +2166,7 @@ int enqueue_persistent(ytrc_batch *b, hipStream_t s)
         HIPCHK(hipEventRecord(b->ev_join, b->ctx->stream2));
         HIPCHK(hipStreamWaitEvent(s, b->ev_join, 0));
     }
+    unjoined.armed = false;
     return YTRC_OK;
 }
 
