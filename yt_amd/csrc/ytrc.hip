@@ -223,7 +223,8 @@ namespace {
 // Kernel variant of a request: KIND, interleaved fields NFP, record mode and
 // MODE (VR: bit 0 ColorTransferFunction path, bit 1 n_samples == 10, bit 2
 // early ray termination, bit 3 per-pixel lens, bit 4 vertex blocks in LDS,
-// bit 5 with bit 0 grey opacity (one field, no bit 2); projection: bit 3).
+// bit 5 with bit 0 grey opacity (one field, no bit 2); projection: bit 3,
+// bit 6 by the launch: more_waves).
 // NFP 4 and 8 variants keep only bits 0 and 3.
 // Sampler kinds that read a transfer function.
 inline bool has_tf(int kind) { return kind == YTRC_VOLUME_RENDER || kind == YTRC_LIGHT_SOURCE; }
@@ -394,6 +395,22 @@ pfn_t split_kernel(int n_cu, int kind, int nfp, bool rec, int mode, int n_order,
     if (nfp != 1 || rec) return nullptr;
     const double most = n_order == 1 ? 1.25 : 0.75;
     return chains <= most * 4.0 * n_cu ? pick_split(kind, mode) : nullptr;
+}
+
+// Mode bit 6 for a launch of n tiles: the two-field projection kernel of 4
+// waves per SIMD (MinWaves), whose few spilled registers cost every tile a
+// little, instead of 3 without spills.  Time of 3 over time of 4, weighted
+// projections of 96^3 / 192^3 / 256^3 / 192^3 in 8 bricks / 200^3 in 64:
+//   1024^2 (64 tiles per CU)  1.03 / 1.09 / 1.11 / 1.11 / 1.12
+//   724^2 (32)                0.93 / 1.02 / 1.02 / 1.03 / 1.05
+//   512^2 (16)                0.94 / 1.05 / 1.11 / 0.91 / 0.90
+//   256^2 (4)                 0.98 / 1.01 / 0.99 / 0.98 / 0.99
+// It is taken where the slots of 3 waves (12 per CU) are filled more than
+// three times.  The per-pixel kernel loses 1 to 13 % by it below 724^2 and
+// stays at 3.
+int more_waves(int n_cu, int kind, int nfp, bool rec, int mode, int64_t n)
+{
+    return kind == YTRC_PROJECTION && nfp == 2 && !rec && mode == 0 && n > 36 * (int64_t)n_cu ? 64 : 0;
 }
 
 // Words of LDS per wave that a persistent launch gives after its tables
@@ -1944,7 +1961,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         g.nfp = std::get<1>(plans[L].variant);
         g.rec = std::get<2>(plans[L].variant) != 0;
         g.mode = std::get<3>(plans[L].variant);
-        g.fn = pick_persist(g.kind, g.nfp, g.rec, g.mode);
+        g.fn = pick_persist(g.kind, g.nfp, g.rec, g.mode | more_waves(ctx->n_cu, g.kind, g.nfp, g.rec, g.mode, ntiles));
         g.split = g.fn;
         for (int i : ids)
             if (g.split != nullptr)
@@ -2299,7 +2316,8 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
     memset(queue, 0, sizeof(unsigned int) * QCOUNTERS);
     set_bounds(queue, cut);
     memcpy(Ht + (img_off - tf_off), &d, sizeof(DImg));
-    pfn_t fn = pick_persist(req->kind, P.q.nfp, false, P.q.mode);
+    pfn_t fn = pick_persist(req->kind, P.q.nfp, false,
+                            P.q.mode | more_waves(ctx->n_cu, req->kind, P.q.nfp, false, P.q.mode, P.q.ntiles));
     if (fn == nullptr) return fail(YTRC_ENOTIMPL, "ytrc_render_noalloc: no kernel for this request");
     const int wpg = 4, threads = 64 * wpg;
     const size_t tables = has_tf(req->kind) ? sizeof(float4) * P.tft.size() : 0;
@@ -2897,14 +2915,16 @@ int srv_pump(ytrc_server *S)
         HIPCHK(hipEventRecord(C.staged, s));
         for (int v = 0; v < nv; v++) {
             if (vcnt[v] == 0) continue;
-            const bool vr = has_tf(std::get<0>(S->vkeys[v]));
-            const int ww = required_wave_words(std::get<0>(S->vkeys[v]), std::get<1>(S->vkeys[v]),
-                                               std::get<2>(S->vkeys[v]) != 0, std::get<3>(S->vkeys[v]));
+            const auto [kind, nfp, record, mode] = S->vkeys[v];
+            const bool vr = has_tf(kind);
+            const int more = more_waves(S->ctx->n_cu, kind, nfp, record != 0, mode, vcnt[v]);
+            const pfn_t fn = more ? pick_persist(kind, nfp, record != 0, mode | more) : S->vfns[v];
+            const int ww = required_wave_words(kind, nfp, record != 0, mode);
             const size_t lds = (vr ? sizeof(float4) * S->tf_hi : 0) + 4 * (size_t)ww * sizeof(unsigned);
             int nb = 0;
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, S->vfns[v], 256, lds));
+            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, 256, lds));
             const int grid = std::max(1, std::min(std::max(1, nb) * S->ctx->n_cu, (vcnt[v] + 3) / 4));
-            hipLaunchKernelGGL(S->vfns[v], dim3(grid), dim3(256), lds, s, (const DImg *)S->d_slots,
+            hipLaunchKernelGGL(fn, dim3(grid), dim3(256), lds, s, (const DImg *)S->d_slots,
                                (const int2 *)(C.d_items + voff[v]), C.d_counters + (size_t)v * QCOUNTERS,
                                (const float4 *)S->d_tf, vr ? S->tf_hi : 0, ww);
             HIPCHK(hipGetLastError());

@@ -48,6 +48,7 @@ pfn_t pick_persist_proj(int nfp, bool rec, int mode)
     switch (mode) {
     case 0: return variant_p<0, 0>(nfp, rec);
     case 8: return variant_p<0, 8>(nfp, rec);
+    case 64: return nfp == 2 && !rec ? k_persist<0, 2, false, 64> : nullptr;
     default: return nullptr;
     }
 }

@@ -1902,15 +1902,16 @@ constexpr int QLO = 32, QHI = 33;
 //   slower;
 // - projection, one field, no record: 3.6 % faster than the 5 waves its
 //   90 VGPRs give;
-// - projection, two fields (item x weight and weight): 4 (128 VGPRs) instead
-//   of the 3 its 131 give: 256^3 at 1024^2 0.416 -> 0.373 ms, 64 bricks of
-//   50^3 at 500x700 0.260 -> 0.229; 5 waves 0.377 and 0.248;
+// - projection, two fields (item x weight and weight), in large launches
+//   (MODE bit 6, more_waves): 4 (128 VGPRs, spills outside the visit loop)
+//   instead of the 3 its 135 give: 256^3 at 1024^2 0.416 -> 0.373 ms, 64
+//   bricks of 50^3 at 1024^2 0.556 -> 0.451; 5 waves were slower;
 // - projection, three or four fields: 3 (168 VGPRs); its 169 gave 2, and
 //   three fields of 192^3 at 1024^2 took 0.415 ms, now 0.338.
 template <int KIND, int NFP, bool REC, int MODE>
 struct MinWaves {
     static constexpr bool one = NFP == 1 && !REC;
-    static constexpr int value = (KIND == 0 && NFP == 2 && !REC)                          ? 4
+    static constexpr int value = (KIND == 0 && (MODE & 64) != 0)                          ? 4
                                  : (KIND == 0 && NFP == 4 && !REC && MODE == 0)           ? 3
                                  : !one                                                   ? 1
                                  : (KIND == 1 && (MODE == 1 || MODE == 3 || MODE == 19)) ? 6

@@ -12,7 +12,7 @@ typedef void (*kfn_t)(const DImg *, int);
 
 // Each returns the variant for (nfp, rec, mode) within its unit's family,
 // or nullptr.  Families: projection, interpolated projection and light-source
-// rendering (modes 0, 8); volume rendering modes
+// rendering (modes 0, 8; projection 64: two fields); volume rendering modes
 // 0-1, 2-3, 4-7 (early ray termination), 8-11 (per-pixel lens), 33, 35, 41
 // and 43 (grey opacity).
 pfn_t pick_persist_proj(int nfp, bool rec, int mode);
