@@ -1901,7 +1901,9 @@ constexpr int QLO = 32, QHI = 33;
 // - the same with grey opacity: 4 (128 VGPRs); 5 and 6 waves were 0 to 9 %
 //   slower;
 // - projection, one field, no record: 3.6 % faster than the 5 waves its
-//   90 VGPRs give;
+//   90 VGPRs give; per-pixel lens: 5 (102 VGPRs; 6 spilled inside the visit
+//   loop), perspective 192^3 at 1024^2 0.232 -> 0.212 ms, in 8 bricks 0.270
+//   -> 0.235;
 // - projection, two fields (item x weight and weight), in large launches
 //   (MODE bit 6, more_waves): 4 (128 VGPRs, spills outside the visit loop)
 //   instead of the 3 its 135 give: 256^3 at 1024^2 0.416 -> 0.373 ms, 64
@@ -1916,6 +1918,7 @@ struct MinWaves {
                                  : !one                                                   ? 1
                                  : (KIND == 1 && (MODE == 1 || MODE == 3 || MODE == 19)) ? 6
                                  : (KIND == 1 && (MODE & 32) != 0)                       ? 4
+                                 : (KIND == 0 && MODE == 8)                              ? 5
                                  : (KIND == 0)                                           ? 6
                                                                                          : 1;
 };
