@@ -263,7 +263,8 @@ std::vector<int> tiles_z_order(int tiles0, int tiles1)
 // The estimated cost of each ray tile of one request, relative: the longest
 // chord of the rays at the tile's corners (plane-parallel lens) or centre
 // through the box around its bricks, plus 1/32 of that box's longest chord
-// for the tile itself.  Only the queue's order depends on it.
+// for the tile itself.  The queue's order and the waves to a tile depend on
+// it, no value does.
 std::vector<float> tile_costs(const ytrc_request &r, const DBrick *bricks, int tsh)
 {
     const int th = 64 >> tsh, tw = 1 << tsh;
@@ -352,18 +353,36 @@ void set_bounds(unsigned int *queue, const int cut[QSPLIT + 1])
 // The step (0 .. 15) of a tile's cost in the costly-first order.
 int cost_step(float cost, float most) { return std::min(15, (int)(16.0f * cost / most)); }
 
-// Whether a launch of n single-tile items takes its costly tiles first.  It
-// evens out the SIMDs where few items follow the first ones; with more of
-// them the queue does, and the Z order keeps lines in L2.  Measured, kernel
-// time in launch order -> costly first: 256^3 volume render at 800x600 (1.2
-// items per slot) 1.02 -> 0.88 ms, 192^3 grey at 512^2 (0.7) 1.01 -> 0.87,
-// perspective 501x333 (0.4) 0.435 -> 0.413, 1672-brick render at 1024^2 (2.7)
-// 1.55 -> 1.55; projections, held by memory, 64 bricks at 500x700 (0.9) 0.224
-// -> 0.205, but 256^3 at 1024^2 (2.7) 0.379 -> 0.391.
-bool few_items(int n_cu, int kind, int64_t n)
+// Whether a launch of n single-tile items, of requests of up to n_order
+// bricks, cuts its images by cost and takes their costly tiles first.  That
+// evens out the SIMDs and XCDs where few items follow the first ones; with
+// more of them the queue does, and runs of equal length in Z order keep lines
+// in L2.  Kernel times in that order -> by cost:
+// - volume renders, per wave slot (24 per CU) that the launch has items: 256^3
+//   at 800x600 (1.2 items) 1.02 -> 0.88 ms, 192^3 grey at 512^2 (0.7) 1.01 ->
+//   0.87, perspective 501x333 (0.4) 0.435 -> 0.413, 192^3 at 1024^2 (2.7) 1.59
+//   -> 1.42; above 4 items no faster.  With four waves to a tile also where
+//   all tiles start at once: 192^3 at 256^2 0.30 -> 0.27.
+// - interpolated projections, 192^3 at 1024^2 0.72 -> 0.67, perspective 256^3
+//   0.66 -> 0.59, 96^3 perspective 0.275 -> 0.285; up to one wave per SIMD (4
+//   per CU) 2 to 4 % slower.
+// - projections, held by memory: 64 bricks at 500x700 (0.9) 0.224 -> 0.205;
+//   one brick, by size and camera 0.84 to 1.14 of the time it had: 192^3 at
+//   512^2 0.134 -> 0.123, but perspective 0.100 -> 0.114 (two fields), 96^3
+//   at 724^2 0.137 -> 0.155, and above one item per slot 192^3 perspective at
+//   1024^2 0.231 -> 0.260.
+bool few_items(int n_cu, int kind, int64_t n, int n_order)
 {
     const int64_t slots = (int64_t)n_cu * 24;  // at 6 waves per SIMD
-    return n < (kind == YTRC_PROJECTION ? slots : 4 * slots);
+    if (kind == YTRC_VOLUME_RENDER) return n < 4 * slots;
+    if (n <= 4 * (int64_t)n_cu) return false;
+    return kind == YTRC_PROJECTION ? n_order > 1 && n < slots : n < 4 * slots;
+}
+
+// Runs of equal length: cut[0 .. QSPLIT].
+void equal_runs(int n, int cut[QSPLIT + 1])
+{
+    for (int r = 0; r <= QSPLIT; r++) cut[r] = (int)((int64_t)r * n / QSPLIT);
 }
 
 // How many of an image's longest chains of visits all its tiles' chains make
@@ -1873,28 +1892,41 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
     }
     const size_t tfall_off = off;
     off = align_up(off + sizeof(float4) * std::max<size_t>(1, tf_all.size()), 256);
-    // Each image's tiles are cut into QSPLIT contiguous runs of equal
-    // estimated cost and run r goes to queue range r (the range one XCD
-    // drains first), so every XCD renders a compact part of every image and
-    // has the same work: with runs of equal length, the XCDs of an image's
-    // middle had up to twice the work of those of its rim, all of it already
-    // in flight when the others ran dry (256^3 in an 800x600 view: 2.1 of 6
-    // waves per SIMD resident on average).  Within a range the images advance
-    // together (items ordered by the fraction of their run's cost done,
-    // larger images first on ties).  Waves of small images, whose rays are
+    // Each image's tiles are cut into QSPLIT contiguous runs and run r goes
+    // to queue range r (the range one XCD drains first), so every XCD renders
+    // a compact part of every image.  Within a range the images advance
+    // together (items ordered by the fraction of their run done, larger
+    // images first on ties).  Waves of small images, whose rays are
     // sparser than the cells and wait on memory, then run beside waves of
     // large images, which keep the VALUs busy: 5-6 % faster than running
     // the images one after another, larger first.
-    // A launch with few items per wave slot (few_items) takes each range's
-    // costly tiles first instead, in 16 steps of cost and Z order within a
-    // step: nearly all its items are in flight at once, and waves start
-    // SIMD after SIMD, so each SIMD gets its share of every step.
+    // A launch with few items per wave slot (few_items) has nearly all of
+    // them in flight at once.  Its runs have equal estimated cost: with equal
+    // length, the XCDs of an image's middle had up to twice the work of those
+    // of its rim (256^3 in an 800x600 view: 2.1 of 6 waves per SIMD resident
+    // on average).  And it takes each range's costly tiles first, in 16 steps
+    // of cost and Z order within a step: waves start SIMD after SIMD, so each
+    // SIMD gets its share of every step.
     std::vector<std::vector<int2>> gitems;
     std::vector<std::array<int, QSPLIT + 1>> gbounds;
     std::vector<size_t> gitems_off;
+    // the launches that go by cost, and whether any may share tiles
+    std::vector<char> by_cost(plans.size(), 0);
+    bool any_cost = false;
+    for (size_t L = 0; L < plans.size() && (batch_flags & YTRC_BATCH_PERSISTENT); L++) {
+        const auto [kind, nfp, record, mode] = plans[L].variant;
+        int64_t ntiles = 0;
+        int most_bricks = 0;
+        for (int i : plans[L].ids) {
+            ntiles += P[i].q.ntiles;
+            most_bricks = std::max(most_bricks, (int)P[i].q.r.n_order);
+        }
+        by_cost[L] = per_item == 1 && few_items(ctx->n_cu, kind, ntiles, most_bricks);
+        any_cost = any_cost || by_cost[L] || split_kernel(ctx->n_cu, kind, nfp, record != 0, mode, 1, 0.0) != nullptr;
+    }
     std::vector<std::vector<float>> costs((size_t)n_req);
     double chains_all = 0.0;  // the launches run side by side
-    for (int i = 0; i < n_req; i++) {
+    for (int i = 0; i < n_req && any_cost; i++) {
         costs[(size_t)i] = tile_costs(reqs[i], ctx->datasets[reqs[i].ds_id].h_bricks.data(), P[i].tsh);
         chains_all += chains(costs[(size_t)i]);
     }
@@ -1917,7 +1949,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         const bool z = per_item == 1;
         int64_t ntiles = 0;
         for (int i : ids) ntiles += P[i].q.ntiles;
-        const bool costly_first = z && few_items(ctx->n_cu, std::get<0>(plans[L].variant), ntiles);
+        const bool costly_first = by_cost[L] != 0;
         std::vector<std::vector<int>> zord(ids.size());
         std::vector<const float *> cost(ids.size());
         std::vector<float> most(ids.size());
@@ -1926,6 +1958,10 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
             const PrepReq &Q = P[ids[o]];
             const int th = 64 >> Q.tsh, tw = 1 << Q.tsh;
             if (z) zord[o] = tiles_z_order((Q.q.r.nv[0] + th - 1) / th, (Q.q.r.nv[1] + tw - 1) / tw);
+            if (!costly_first) {
+                equal_runs(Q.q.ntiles, cut[o].data());
+                continue;
+            }
             const std::vector<float> &c = costs[(size_t)ids[o]];
             cost[o] = c.data();
             most[o] = *std::max_element(c.begin(), c.end());
@@ -1937,17 +1973,14 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
             for (size_t o = 0; o < ids.size(); o++) {
                 const int i = ids[o];
                 const int t0 = cut[o][(size_t)r], t1 = cut[o][(size_t)r + 1];
-                double total = 0.0, done = 0.0;
-                for (int t = t0; t < t1; t++) total += cost[o][(size_t)(z ? zord[o][(size_t)t] : t)];
                 // an item: up to per_item consecutive tiles, the count in
                 // the top 8 bits of its tile field
                 for (int t = t0; t < t1; t += per_item) {
                     const int cnt = std::min(per_item, t1 - t);
                     const int tile = z ? zord[o][(size_t)t] : t;
                     const double key = costly_first ? (double)-cost_step(cost[o][(size_t)tile], most[o])
-                                                    : done / total;
+                                                    : (double)(t - t0) / (double)(t1 - t0);
                     ks.push_back({key, (int)o, make_int2(i, tile | (cnt << 24))});
-                    for (int q = 0; q < cnt; q++) done += cost[o][(size_t)(z ? zord[o][(size_t)(t + q)] : t + q)];
                 }
             }
             std::stable_sort(ks.begin(), ks.end(), [](const Key &a, const Key &b) {
@@ -1962,7 +1995,7 @@ int ytrc_batch_create(ytrc_ctx *ctx, int32_t n_req, const ytrc_request *reqs,
         g.rec = std::get<2>(plans[L].variant) != 0;
         g.mode = std::get<3>(plans[L].variant);
         g.fn = pick_persist(g.kind, g.nfp, g.rec, g.mode | more_waves(ctx->n_cu, g.kind, g.nfp, g.rec, g.mode, ntiles));
-        g.split = g.fn;
+        g.split = any_cost ? g.fn : nullptr;
         for (int i : ids)
             if (g.split != nullptr)
                 g.split = split_kernel(ctx->n_cu, g.kind, g.nfp, g.rec, g.mode, P[i].q.r.n_order, chains_all);
@@ -2290,16 +2323,20 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
     const bool direct = sizeof(float) * (size_t)P.q.npix * P.q.nch_out <= PIN_OUT;
     if (direct) d.out = (float *)(ctx->pin + PIN_BYTES);
     if (!P.tft.empty()) memcpy(Ht, P.tft.data(), sizeof(float4) * P.tft.size());
-    // One request: the tiles in row order, cut into QSPLIT runs of equal
-    // cost; with few of them, costly ones first within a run, as in a batch.
+    // One request: the tiles in row order, cut into QSPLIT runs; with few of
+    // them, runs of equal cost and the costly tiles first, as in a batch.
     int2 *items = (int2 *)(Ht + (items_off - tf_off));
     int cut[QSPLIT + 1];
     double nchains = 0.0;
     {
-        const std::vector<float> cost = tile_costs(*req, ctx->datasets[req->ds_id].h_bricks.data(), P.tsh);
-        equal_cost_runs(cost, {}, cut);
-        nchains = chains(cost);
-        if (few_items(ctx->n_cu, req->kind, P.q.ntiles)) {
+        const bool by_cost = few_items(ctx->n_cu, req->kind, P.q.ntiles, req->n_order);
+        std::vector<float> cost;
+        if (by_cost || split_kernel(ctx->n_cu, req->kind, P.q.nfp, false, P.q.mode, 1, 0.0) != nullptr) {
+            cost = tile_costs(*req, ctx->datasets[req->ds_id].h_bricks.data(), P.tsh);
+            nchains = chains(cost);
+        }
+        if (by_cost) {
+            equal_cost_runs(cost, {}, cut);
             const float most = *std::max_element(cost.begin(), cost.end());
             for (int r = 0; r < QSPLIT; r++) {
                 int at[17] = {0};
@@ -2309,6 +2346,7 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
                     items[(size_t)(cut[r] + at[15 - cost_step(cost[(size_t)t], most)]++)] = make_int2(0, t);
             }
         } else {
+            equal_runs(P.q.ntiles, cut);
             for (int t = 0; t < P.q.ntiles; t++) items[(size_t)t] = make_int2(0, t);
         }
     }
