@@ -2207,8 +2207,9 @@ int enqueue_persistent(ytrc_batch *b, hipStream_t s)
         }
         g.grid = std::max(1, std::min(per_cu * b->ctx->n_cu,
                                       (g.n_items + per_group - 1) / per_group));
+        unsigned int *queue = b->counters + (size_t)g.counter * QCOUNTERS;
         hipLaunchKernelGGL(fn, dim3(g.grid), dim3(threads), lds, gs, (const DImg *)b->d_imgs,
-                           g.items, b->counters + (size_t)g.counter * QCOUNTERS, b->tf_all + g.tf_base,
+                           g.items, queue, (const unsigned int *)queue, b->tf_all + g.tf_base,
                            g.tf_bins, ww);
         HIPCHK(hipGetLastError());
     }
@@ -2387,7 +2388,7 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
         const int per_group = split ? 1 : wpg;  // tiles at a time
         const int grid = std::max(1, std::min(std::max(1, nb) * ctx->n_cu, (P.q.ntiles + per_group - 1) / per_group));
         hipLaunchKernelGGL(fn, dim3(grid), dim3(threads), lds, s, (const DImg *)(S + img_off),
-                           (const int2 *)(S + items_off), counters,
+                           (const int2 *)(S + items_off), counters, (const unsigned int *)counters,
                            (const float4 *)(S + tf_off), (int)P.tft.size(), ww);
         HIPCHK(hipGetLastError());
     }
@@ -2962,8 +2963,9 @@ int srv_pump(ytrc_server *S)
             int nb = 0;
             HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, 256, lds));
             const int grid = std::max(1, std::min(std::max(1, nb) * S->ctx->n_cu, (vcnt[v] + 3) / 4));
+            unsigned int *queue = C.d_counters + (size_t)v * QCOUNTERS;
             hipLaunchKernelGGL(fn, dim3(grid), dim3(256), lds, s, (const DImg *)S->d_slots,
-                               (const int2 *)(C.d_items + voff[v]), C.d_counters + (size_t)v * QCOUNTERS,
+                               (const int2 *)(C.d_items + voff[v]), queue, (const unsigned int *)queue,
                                (const float4 *)S->d_tf, vr ? S->tf_hi : 0, ww);
             HIPCHK(hipGetLastError());
         }

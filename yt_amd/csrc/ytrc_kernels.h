@@ -1803,17 +1803,23 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
     // wave takes the hits from the ballot, one vector load for 64 extents
     // instead of a scalar load, wait and branch for each.  On an AMR set a
     // tile meets a few dozen of hundreds of bricks, and waves spent 69 % of
-    // their time waiting: 617 bricks at 700x500 took 0.385 ms, now 0.267
-    // (projection); 1672 bricks at 1024^2 2.23 ms, now 1.62 (volume render).
+    // their time waiting: projection of 617 bricks (128^3 and three levels) at
+    // 700x500 0.585 -> 0.479 ms; volume render of 1668 bricks at 1024^2 2.61
+    // -> 1.94.  One brick is the list itself: the ballot's load and wait for
+    // it cost 1 us a tile, 2 % of a small projection.
     for (int base = 0; base < im.n_order; base += 64) {
-        const int kk = base + lane;
-        bool hit = false;
-        if (kk < im.n_order) {
-            const int4 e = im.ext[ert ? im.n_order - 1 - kk : kk];
-            hit = !(e.y <= ti0 || e.x >= ti0 + th || e.w <= tj0 || e.z >= tj0 + tw);
+        uint64_t hits = 1;
+        if (im.n_order > 1) {
+            const int kk = base + lane;
+            bool hit = false;
+            if (kk < im.n_order) {
+                const int4 e = im.ext[ert ? im.n_order - 1 - kk : kk];
+                hit = !(e.y <= ti0 || e.x >= ti0 + th || e.w <= tj0 || e.z >= tj0 + tw);
+            }
+            hits = __ballot(hit);
         }
         bool done = false;
-        for (uint64_t hits = __ballot(hit); hits != 0 && !done; hits &= hits - 1) {
+        for (; hits != 0 && !done; hits &= hits - 1) {
             const int k = base + __builtin_ctzll(hits);
             done = cast_brick(ert ? im.n_order - 1 - k : k);
         }
@@ -1881,7 +1887,8 @@ constexpr int QSPLIT = 8;
 constexpr int QSTRIDE = 64;
 constexpr int QCOUNTERS = QSPLIT * QSTRIDE;  // words of counters per launch
 // The range's first item and the one past its last, on the counter's next
-// line (read, never written, during the launch).
+// line (read, never written, during the launch: the kernels take the same
+// address a second time as read-only memory, for scalar loads).
 constexpr int QLO = 32, QHI = 33;
 
 // Persistent launch: every wave repeatedly takes the next (image, tile)
@@ -1928,6 +1935,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MinWaves<KI
 void k_persist(const DImg *__restrict__ imgs,
                                                  const int2 *__restrict__ items,
                                                  unsigned int *__restrict__ counter,
+                                                 const unsigned int *__restrict__ bounds,
                                                  const float4 *__restrict__ tf_all, int tf_bins, int wave_words)
 {
     extern __shared__ float4 s_tf[];
@@ -1955,8 +1963,7 @@ void k_persist(const DImg *__restrict__ imgs,
         unsigned int it = 0;
         if (lane == 0) it = atomicAdd(counter + part * QSTRIDE, 1u);
         it = (unsigned int)__builtin_amdgcn_readfirstlane((int)__shfl(it, 0));
-        const unsigned int lo = (unsigned int)uni((int)counter[part * QSTRIDE + QLO]);
-        const unsigned int hi = (unsigned int)uni((int)counter[part * QSTRIDE + QHI]);
+        const unsigned int lo = bounds[part * QSTRIDE + QLO], hi = bounds[part * QSTRIDE + QHI];
         if (it >= hi - lo) {
             if (--left == 0) break;
             part = (part + 1 == QSPLIT) ? 0 : part + 1;
@@ -1996,7 +2003,7 @@ void k_persist(const DImg *__restrict__ imgs,
 template <int MODE>
 __global__ __launch_bounds__(64 * NSEG) __attribute__((amdgpu_waves_per_eu(4)))
 void k_split(const DImg *__restrict__ imgs, const int2 *__restrict__ items, unsigned int *__restrict__ counter,
-             const float4 *__restrict__ tf_all, int tf_bins, int)
+             const unsigned int *__restrict__ bounds, const float4 *__restrict__ tf_all, int tf_bins, int)
 {
     extern __shared__ float4 s_tf[];
     for (int i = threadIdx.x; i < tf_bins; i += blockDim.x) s_tf[i] = tf_all[i];
@@ -2012,7 +2019,7 @@ void k_split(const DImg *__restrict__ imgs, const int2 *__restrict__ items, unsi
             int2 w = make_int2(-1, 0);
             while (left > 0) {
                 const unsigned int it = atomicAdd(counter + part * QSTRIDE, 1u);
-                const unsigned int lo = counter[part * QSTRIDE + QLO], hi = counter[part * QSTRIDE + QHI];
+                const unsigned int lo = bounds[part * QSTRIDE + QLO], hi = bounds[part * QSTRIDE + QHI];
                 if (it < hi - lo) {
                     w = items[lo + it];
                     break;
