@@ -1757,6 +1757,7 @@ int read_request_image(ytrc_ctx *ctx, const ReqHost &q, const DImg &d, double *i
     if (q.r.flags & YTRC_FLAG_PARTIAL)
         return fail(YTRC_EINVAL, "a YTRC_FLAG_PARTIAL request has a map, not an image: "
                                  "read it with ytrc_batch_read_partial");
+    constexpr int64_t RUN = 1 << 20;  // pixels a call
     const ImageRun run = image_run(q, image_out);
     // Small images on this thread: the transfer's launches and wake-ups take
     // about 25 us.  One thread takes 0.8 ns a pixel for one channel (34 us
@@ -1764,13 +1765,16 @@ int read_request_image(ytrc_ctx *ctx, const ReqHost &q, const DImg &d, double *i
     // for three merged with an input image; where the sum below is larger,
     // several threads are faster (256^2: 49 -> 47, 82 -> 60, 121 -> 71, 126 ->
     // 63 us).
-    if (q.npix * (1 + q.nch_out + (run.in != nullptr ? 4 : 0)) <= 100000) {
+    // And images that find the transfer busy: several threads that read at
+    // once have their own copies and conversions side by side (8 of 512^2:
+    // 0.64 ms each; in line for the transfer 0.88).
+    std::unique_lock<std::mutex> lk(ctx->xfer.mu, std::defer_lock);
+    if (q.npix * (1 + q.nch_out + (run.in != nullptr ? 4 : 0)) <= 100000 || !lk.try_lock()) {
         std::vector<float> h((size_t)q.npix * q.nch_out);
         HIPCHK(hipMemcpy(h.data(), d.out, sizeof(float) * h.size(), hipMemcpyDeviceToHost));
-        run(0, (int)q.npix, h.data(), q.npix);
+        for (int64_t at = 0; at < q.npix; at += RUN) run(at, (int)std::min(RUN, q.npix - at), h.data() + at, q.npix);
         return YTRC_OK;
     }
-    std::lock_guard<std::mutex> lk(ctx->xfer.mu);
     HIPCHK(ctx->xfer.read(ctx->xfer.stream, d.out, q.npix, q.nch_out, image_out, 4 * sizeof(double), run));
     return YTRC_OK;
 }
@@ -2406,8 +2410,8 @@ int ytrc_render_noalloc(ytrc_ctx *ctx, const ytrc_request *req, double *image_ou
     }
     HIPCHK(hipStreamSynchronize(s));
     if (!direct) return read_request_image(ctx, P.q, d, image_out);
-    std::lock_guard<std::mutex> lx(ctx->xfer.mu);
-    ctx->xfer.read_here(d.out, P.q.npix, image_out, 4 * sizeof(double), image_run(P.q, image_out));
+    std::unique_lock<std::mutex> lx(ctx->xfer.mu, std::try_to_lock);
+    ctx->xfer.read_here(lx.owns_lock(), d.out, P.q.npix, image_out, 4 * sizeof(double), image_run(P.q, image_out));
     return YTRC_OK;
 }
 
@@ -3252,11 +3256,12 @@ int ytrc_server_read_planar(ytrc_server *S, int64_t id, float *planes, int32_t c
     const int64_t count = q.npix * q.nch_out;
     // Small ones in one copy: up to 960 KB it is the faster way (420^2: 39 us,
     // by several threads 54; 512^2 65 and 65), less far with values to merge.
-    if (count * (in != nullptr ? 4 : 1) <= 240000) {
+    // (Or while the transfer is busy, as for images.)
+    std::unique_lock<std::mutex> lx(S->ctx->xfer.mu, std::defer_lock);
+    if (count * (in != nullptr ? 4 : 1) <= 240000 || !lx.try_lock()) {
         HIPCHK(hipMemcpy(planes, it->second.d.out, sizeof(float) * (size_t)count, hipMemcpyDeviceToHost));
         merge(0, count);
     } else {
-        std::lock_guard<std::mutex> lx(S->ctx->xfer.mu);
         HIPCHK(S->ctx->xfer.read(S->ctx->xfer.stream, it->second.d.out, count, 1, planes, sizeof(float),
                                  [&merge, planes](int64_t first, int n, const float *from, int64_t) {
                                      memcpy(planes + first, from, sizeof(float) * (size_t)n);

@@ -128,7 +128,7 @@ class Helpers {
 };
 
 // A context's pinned buffers and helper threads.  One transfer at a time:
-// `mu` is held by each.
+// `mu` is held by each; callers that find it taken copy by themselves.
 class Transfer {
   public:
     struct Piece {
@@ -215,11 +215,12 @@ class Transfer {
         return hipSuccess;
     }
 
-    // read() of planes of npix floats that are in host memory already.
+    // read() of planes of npix floats that are in host memory already; by the
+    // calling thread alone where it does not hold `mu`.
     template <class F>
-    void read_here(const float *planes, int64_t npix, const void *out, size_t px_bytes, F &&each)
+    void read_here(bool held, const float *planes, int64_t npix, const void *out, size_t px_bytes, F &&each)
     {
-        convert(planes, npix, npix, (const char *)out, px_bytes, each);
+        convert(planes, npix, npix, (const char *)out, px_bytes, each, held);
     }
 
     // Copies the pieces, one after another, to dst on the device in order of
@@ -282,7 +283,8 @@ class Transfer {
     // array: threads that fault on one page at once each clear 2 MB for it
     // and all but one throw it away.  Small arrays have small pages.
     template <class F>
-    void convert(const float *planes, int64_t stride, int64_t count, const char *out, size_t px_bytes, F &&each)
+    void convert(const float *planes, int64_t stride, int64_t count, const char *out, size_t px_bytes, F &&each,
+                 bool helped = true)
     {
         const size_t bytes = (size_t)count * px_bytes;
         const size_t page = bytes >= 2 * PAGE ? PAGE : PAGE / 8;
@@ -299,7 +301,10 @@ class Transfer {
                 each(a, (int)(b - a), planes + a, stride);
             }
         };
-        helpers_->run(nu - 1, job);
+        if (helped)
+            helpers_->run(nu - 1, job);
+        else
+            job();
     }
 
     // Waits until the copy engine has taken half h.
