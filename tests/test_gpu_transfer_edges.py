@@ -1,8 +1,9 @@
 """Images at the sizes where the way they travel changes: one thread's copy
 and the pinned transfer (by pixels and channels), the transfer's parts (256 KiB
 to a quarter of an image, five where the count is no multiple of 16) and its 12
-MiB window, and render_noalloc's 4 MiB of output in pinned memory.  Bar: every
-value bit for bit.
+MiB window, and render_noalloc's 4 MiB of output in pinned memory; and uploads
+on either side of the rule that copies them as they are or through the pinned
+windows.  Bar: every value bit for bit.
 """
 
 import numpy as np
@@ -11,6 +12,7 @@ import pytest
 from yt_amd import _lib, render
 
 from .helpers import c0_params, uniform_lognormal, vr_tf_for
+from .test_gpu_transfer import _blocked
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +79,37 @@ def test_images_at_the_edges(ctx, volume, kind, nch, n):
             assert nv[0] == 1 or np.any(image != 0)
             assert np.array_equal(served, image) and np.array_equal(direct, image)
             assert np.array_equal(planes, np.moveaxis(image[..., :nch], -1, 0).astype(np.float32))
+
+
+# one piece on either side of 16 and 48 KiB and of 3 MiB, two pieces below, at and above 128 KiB
+# and 3 MiB in all, three pieces
+@pytest.mark.parametrize("dims,nf,dtype", [
+    ([(1, 3, 5)], 1, np.float64),
+    ([(16, 16, 15)], 1, np.float32),
+    ([(16, 16, 16)], 1, np.float32),
+    ([(16, 16, 24)], 1, np.float64),
+    ([(16, 17, 24)], 1, np.float64),
+    ([(96, 64, 127)], 1, np.float32),
+    ([(96, 64, 128)], 1, np.float32),
+    ([(3, 65536, 2)], 1, np.float64),
+    ([(96, 64, 129)], 1, np.float32),
+    ([(32, 32, 16)], 2, np.float32),
+    ([(16, 32, 16), (16, 32, 16)], 1, np.float64),
+    ([(32, 32, 16), (32, 33, 16)], 1, np.float32),
+    ([(64, 64, 47), (64, 64, 48)], 1, np.float64),
+    ([(64, 64, 48), (64, 64, 48)], 1, np.float64),
+    ([(64, 64, 49), (64, 64, 49)], 1, np.float64),
+    ([(31, 17, 9)], 3, np.float64),
+])
+def test_uploads_at_the_edges(ctx, dims, nf, dtype):
+    print(f"upload edge: {dims} {nf} {dtype.__name__}", flush=True)
+    rng = np.random.default_rng(nf)
+    bricks = [((k, 0.0, 0.0), (k + 1.0, 1.0, 1.0), d, False) for k, d in enumerate(dims)]
+    fields = [[rng.standard_normal(d).astype(dtype) for _ in range(nf)] for d in dims]
+    for _ in range(2):
+        ds = ctx.upload(bricks, fields)
+        try:
+            for b in range(len(dims)):
+                assert np.array_equal(ctx.read_points(ds, b), _blocked(fields[b])), b
+        finally:
+            ctx.free(ds)

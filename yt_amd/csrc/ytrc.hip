@@ -1048,11 +1048,7 @@ int ytrc_dataset_upload(ytrc_ctx *ctx, int32_t n_bricks, const ytrc_brick_desc *
         return hipGetLastError();
     };
     auto flush = [&]() -> hipError_t {
-        hipError_t er;
-        {
-            std::lock_guard<std::mutex> lx(ctx->xfer.mu);
-            er = ctx->xfer.write(ctx->stream, pieces, stg.p);
-        }
+        hipError_t er = ctx->xfer.write(ctx->stream, pieces, stg.p);
         for (const Field &g : group)
             if (er == hipSuccess) er = store(g.b, g.f, stg.p + g.at);
         group.clear();
@@ -1151,7 +1147,6 @@ int ytrc_dataset_build_vr(ytrc_ctx *ctx, int32_t n_grids, const ytrc_grid_desc *
             for (int f = 0; f < n_fields; f++)
                 pieces.push_back({(const char *)cell_ptrs[(size_t)g * n_fields + f], nc * esz});
         }
-        std::lock_guard<std::mutex> lx(ctx->xfer.mu);
         e = ctx->xfer.write(ctx->stream, pieces, stg.p);
     }
     if (e != hipSuccess) return bail(e, "hipMemcpyAsync(cells)");
