@@ -1,8 +1,9 @@
 """Images and fields through the pinned transfer buffers.
 
-Read-back moves chunks of 4096 pixels through two 4 MiB halves; uploads move
-windows of at most 4 MiB, and fields are staged up to 32 MiB at a time.  The
-sizes here lie at the edges of those.  Bar: every value bit for bit.
+Read-back moves planes through a 12 MiB buffer, in quarters; uploads move
+windows of at most 4 MiB, and fields are staged up to 32 MiB at a time.  Sizes
+from one pixel and one cell to more than those; the exact edges are
+test_gpu_transfer_edges.py's.  Bar: every value bit for bit.
 
 * An image that no ray of a volume render touches comes back as the input
   image: the device holds its float32 values, and a pixel whose value went

@@ -407,8 +407,10 @@ double chains(const std::vector<float> &cost)
 //   one brick       0.1 to 0.6: 1.3 to 2.0, 0.9: 1.15 to 1.34, 1.3: 1.08 to
 //                   1.11, 1.8: 0.87 to 1.26, 2.1: 0.87
 //   per-pixel lens  0.2: 1.5 to 2.1, 0.8: 1.2 to 1.34, 1.3: 1.02 to 1.2, 2.0: 0.84
-//   more bricks     (whose rays' ends fill rounds badly) 0.2: 1.4 to 1.8, 0.5:
-//                   1.41, 0.6: 1.38, 0.9: 1.07 to 1.11, 1.2: 0.89
+//   more bricks     (whose rays' ends fill rounds badly) 0.2: 1.4 to 1.9, 0.5:
+//                   1.4 to 1.8, 0.7: 1.25 to 1.7, 0.9: 1.07 to 1.6, 1.2: 0.89
+//                   to 1.6, 1.8: 0.8 to 1.4 (8 and 64 bricks, AMR sets of
+//                   some hundred and of 1668; perspective the same)
 pfn_t split_kernel(int n_cu, int kind, int nfp, bool rec, int mode, int n_order, double chains)
 {
     if (nfp != 1 || rec) return nullptr;
@@ -1469,13 +1471,13 @@ int prep_request(ytrc_ctx *ctx, const ytrc_request &r, const std::string &tag, P
             q.tform = bounded && (emax * (tcell / (double)r.n_samples) * 1.001 <= 1.0);
         }
         // ColorTransferFunction pattern (transfer_functions.py:385-408) in
-        // transmittance form gets its own kernel path (MODE bit 0); grey or
-        // unbounded CTFs take the general per-table path.
-        // Grey opacity on one field without early termination or partial maps
-        // gets its own layout and compositing (MODE bits 0 and 5,
-        // ctf_visit_grey) where dt * alpha <= 1 holds for every sub-sample by
-        // the same bound, so that the reference's clamp of 1 - dt alpha never
-        // acts, and the tables are finite.
+        // transmittance form gets its own kernel path (MODE bit 0); unbounded
+        // CTFs take the general per-table path.  Grey opacity on one field
+        // without early termination or partial maps gets its own layout and
+        // compositing (MODE bits 0 and 5, ctf_visit_grey) where dt * alpha <=
+        // 1 holds for every sub-sample by the same bound, so that the
+        // reference's clamp of 1 - dt alpha never acts, and the tables are
+        // finite; otherwise the general path too.
         const bool grey = ctf && T.grey && r.kind == YTRC_VOLUME_RENDER && q.nfp == 1 &&
                           !(r.flags & (YTRC_FLAG_ERT | YTRC_FLAG_PARTIAL)) && grey_bounded(tf, tcell / (double)r.n_samples);
         ctf = (ctf && q.tform && r.kind == YTRC_VOLUME_RENDER) || grey;

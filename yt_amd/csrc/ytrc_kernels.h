@@ -656,7 +656,7 @@ __device__ __forceinline__ void ctf_visit(const TFCache &tf, const float4 *__res
 // the reference's clamp of 1 - dt alpha at 0 never acts.  k: the value along
 // the visit's sub-samples, k0 + k1 s + k2 s^2 + k3 s^3.  About 20 FP32 and
 // 12 FP64 VALU per sub-sample bound it; with the general tables' 16 lookups'
-// worth of selects, 192^3 at 512^2 took 5.34 ms, now 1.00 ms.
+// worth of selects, 192^3 at 512^2 took 5.34 ms, now 0.90 ms.
 template <int NS>
 __device__ __forceinline__ void ctf_visit_grey(const TFCache &tf, const float4 *__restrict__ lt,
                                                const float (&k)[4], double dt, int ns, double (&st)[4])
@@ -1110,8 +1110,8 @@ struct IProjSampler {
 // walk_vr_ctf_fast's conditions (walk_init left every walking lane inside
 // the brick, vertex blocks below 2^32 bytes, strides of 24 bits): no bounds
 // test per visit, the corners through a buffer resource at a 32-bit offset
-// summed over axes, cell indices also kept as doubles (stepped, exact) for
-// the sample positions, minima by one instruction, the axis step as nested
+// summed over axes, cell indices also kept as doubles (formed from
+// the integers at each step, exact) for the sample positions, minima by one instruction, the axis step as nested
 // branches.  The sampler's arithmetic, and so every value, is that of
 // walk_loop.  SHARED: all rays have one direction (steps and increments are
 // scalar).
@@ -1803,7 +1803,7 @@ __device__ __forceinline__ void render_tile(const DImg &im, int tile, int lane,
     // wave takes the hits from the ballot, one vector load for 64 extents
     // instead of a scalar load, wait and branch for each.  On an AMR set a
     // tile meets a few dozen of hundreds of bricks, and waves spent 69 % of
-    // their time waiting: projection of 617 bricks (128^3 and three levels) at
+    // their time waiting: projection of 619 bricks (128^3 and three levels) at
     // 700x500 0.585 -> 0.479 ms; volume render of 1668 bricks at 1024^2 2.61
     // -> 1.94.  One brick is the list itself: the ballot's load and wait for
     // it cost 1 us a tile, 2 % of a small projection.
@@ -1908,12 +1908,12 @@ constexpr int QLO = 32, QHI = 33;
 // - the same with grey opacity: 4 (128 VGPRs); 5 and 6 waves were 0 to 9 %
 //   slower;
 // - projection, one field, no record: 3.6 % faster than the 5 waves its
-//   90 VGPRs give; per-pixel lens: 5 (102 VGPRs; 6 spilled inside the visit
-//   loop), perspective 192^3 at 1024^2 0.232 -> 0.212 ms, in 8 bricks 0.270
+//   90 VGPRs give; per-pixel lens: 5 (102 VGPRs; at 6 the visit loop
+//   spills), perspective 192^3 at 1024^2 0.232 -> 0.212 ms, in 8 bricks 0.270
 //   -> 0.235;
 // - projection, two fields (item x weight and weight), in large launches
 //   (MODE bit 6, more_waves): 4 (128 VGPRs, spills outside the visit loop)
-//   instead of the 3 its 135 give: 256^3 at 1024^2 0.416 -> 0.373 ms, 64
+//   instead of the 3 its 135 give: 256^3 at 1024^2 0.391 -> 0.353 ms, 64
 //   bricks of 50^3 at 1024^2 0.556 -> 0.451; 5 waves were slower;
 // - projection, three or four fields: 3 (168 VGPRs); its 169 gave 2, and
 //   three fields of 192^3 at 1024^2 took 0.415 ms, now 0.338.
@@ -1992,7 +1992,7 @@ void k_persist(const DImg *__restrict__ imgs,
 // 10 sub-samples for a lone wave, and with a wave per tile the longest
 // chains are the launch's time while the chip is not full (split_kernel).
 // Here a wave samples a quarter of the visits and steps over the others, at
-// 20 of 270 operations each; the rounds' exchange costs 6 operations a visit.
+// 20 of 270 operations each; the rounds' exchange costs 8 operations a visit.
 // One wave a tile -> four, same images: 256^3 at 200^2 0.63 -> 0.32 ms,
 // perspective 160^3 at 501x333 0.45 -> 0.36, at 200^2 0.44 -> 0.23.
 // Measured and not kept: parts of a ray's chain multiplied together (faster,
