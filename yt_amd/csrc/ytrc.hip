@@ -370,7 +370,10 @@ int cost_step(float cost, float most) { return std::min(15, (int)(16.0f * cost /
 //   one brick, by size and camera 0.84 to 1.14 of the time it had: 192^3 at
 //   512^2 0.134 -> 0.123, but perspective 0.100 -> 0.114 (two fields), 96^3
 //   at 724^2 0.137 -> 0.155, and above one item per slot 192^3 perspective at
-//   1024^2 0.231 -> 0.260.
+//   1024^2 0.231 -> 0.260.  Where a large brick's kernel gains (256^3 at
+//   512^2, weighted, 0.163 -> 0.138) the host's estimate of the costs takes
+//   more than that: whole render_noalloc calls of 192^3 and 256^3 at 448^2
+//   to 600^2 take 1.02 to 1.28 times as long by cost, that one 0.273 -> 0.289.
 bool few_items(int n_cu, int kind, int64_t n, int n_order)
 {
     const int64_t slots = (int64_t)n_cu * 24;  // at 6 waves per SIMD
