@@ -373,7 +373,7 @@ int cost_step(float cost, float most) { return std::min(15, (int)(16.0f * cost /
 //   1024^2 0.231 -> 0.260.  Where a large brick's kernel gains (256^3 at
 //   512^2, weighted, 0.163 -> 0.138) the host's estimate of the costs takes
 //   more than that: whole render_noalloc calls of 192^3 and 256^3 at 448^2
-//   to 600^2 take 1.02 to 1.28 times as long by cost, that one 0.273 -> 0.289.
+//   to 600^2 take 1.03 to 1.20 times as long by cost, that one 0.268 -> 0.280.
 bool few_items(int n_cu, int kind, int64_t n, int n_order)
 {
     const int64_t slots = (int64_t)n_cu * 24;  // at 6 waves per SIMD
